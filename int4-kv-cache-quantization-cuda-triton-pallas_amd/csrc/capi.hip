@@ -87,23 +87,18 @@ int pick_heads_per_wg(int d, int hq_per_kv) {
   return 1;
 }
 
-// Kernel family: with two or more q-heads per kv-head at D = 64 or 128 the
-// int8 matrix-core kernel (2, 4 or 8 heads per workgroup, 8 only at D=64;
-// B8 Hkv8 Hq32 T8192: 61 us against 75 us for the vector grouped kernel);
-// with one head per kv-head the vector per-head kernel, which is faster there
-// (anchor 51.9 against 54.2 us). FDI4_TUNE_DECODE_VECTOR_ONLY selects the
-// vector kernels throughout (A/B measurement).
-bool use_mfma(int d) {
-  const bool off = g_tuning[FDI4_TUNE_DECODE_VECTOR_ONLY].load(std::memory_order_relaxed) == 1;
-  return !off && (d == 64 || d == 128);
+// Kernel family: with two or more q-heads per kv-head the matrix-core kernel
+// (2, 4 or 8 heads per workgroup); with one head per kv-head the vector
+// per-head kernel. FDI4_TUNE_DECODE_VECTOR_ONLY selects the vector kernels
+// throughout (A/B measurement).
+bool use_mfma() {
+  return g_tuning[FDI4_TUNE_DECODE_VECTOR_ONLY].load(std::memory_order_relaxed) != 1;
 }
 
-// Up to eight heads per workgroup (at D=128: 248 VGPRs with float32 values,
-// 244 with float16, no spills).
-int pick_heads_per_wg_mfma(int d, int v_dtype, int hq_per_kv) {
-  (void)d;
-  (void)v_dtype;
-  const int cap = heads_per_wg_cap();
+// Up to eight heads per workgroup, four at D = 256 (64 accumulator registers
+// beside 32 of digits and 64 of values in flight).
+int pick_heads_per_wg_mfma(int d, int hq_per_kv) {
+  const int cap = std::min(heads_per_wg_cap(), d == 256 ? 4 : 8);
   for (int hg : {8, 4, 2})
     if (hg <= cap && hq_per_kv % hg == 0) return hg;
   return 1;
@@ -140,14 +135,15 @@ bool one_wave_per_simd(int d, int v_dtype, int64_t streams) {
 // waves that re-quantize the open group meanwhile.
 DecodePlan plan_decode(int batch, int hq, int hq_per_kv, int d, int v_dtype, int chunks) {
   DecodePlan p;
-  p.mfma = use_mfma(d) ? 1 : 0;
-  p.heads_per_wg = p.mfma ? pick_heads_per_wg_mfma(d, v_dtype, hq_per_kv)
+  p.mfma = use_mfma() ? 1 : 0;
+  p.heads_per_wg = p.mfma ? pick_heads_per_wg_mfma(d, hq_per_kv)
                           : pick_heads_per_wg(d, hq_per_kv);
   if (p.heads_per_wg == 1) p.mfma = 0;
   const int64_t streams = (int64_t)batch * (hq / p.heads_per_wg);
   const bool per_simd = !p.mfma && p.heads_per_wg == 1 && one_wave_per_simd(d, v_dtype, streams);
   const int forced = g_tuning[FDI4_TUNE_DECODE_WAVES].load(std::memory_order_relaxed);
-  if (!p.mfma && p.heads_per_wg > 1 && d == 256) p.waves = 4;
+  // Where eight waves of the grouped kernels would spill registers.
+  if (p.heads_per_wg > 1 && d == 256 && (!p.mfma || v_dtype == FDI4_V_F32)) p.waves = 4;
   else if (per_simd && forced == 0) p.waves = 4;
   else p.waves = pick_waves(chunks);
   if (chunks <= 0) {
@@ -556,6 +552,10 @@ int make_decode_args(const void* query, int q_dtype, int batch, int num_q_heads,
   a->max_pages = cache->max_pages;
   a->hq_per_kv = num_q_heads / cache->num_kv_heads;
   a->num_pages = cache->num_pages;
+  a->div_rows = fdi4::make_fast_div(cache->page_rows);
+  a->div_cpp = fdi4::make_fast_div(ceil_div(cache->page_rows, 16));
+  a->div_ppg = fdi4::make_fast_div(cache->pages_per_group);
+  a->div_hpk = fdi4::make_fast_div(a->hq_per_kv);
   a->chunks_per_split = std::max(1, ceil_div(chunks, splits));
   a->num_splits = splits;
   a->num_q_heads = num_q_heads;

@@ -141,7 +141,7 @@ decode_kernel(DecodeArgs a) {
   constexpr int NT = (WAVES + HW) * 64;
 
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int hk = h / a.hq_per_kv;
+  const int hk = fdiv(h, a.div_hpk);
   const int tid = threadIdx.x, lane = tid & 63;
   // The wave index is uniform across the wave; saying so keeps the chunk loop
   // counters in scalar registers and the page-table reads on the scalar unit.

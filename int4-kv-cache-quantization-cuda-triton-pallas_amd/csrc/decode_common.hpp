@@ -88,6 +88,11 @@ __device__ __forceinline__ int ld_ro(const int32_t* p, int64_t i) {
   return ((const __attribute__((address_space(4))) int32_t*)p)[i];
 }
 
+// n / d for the divisor behind f (0 <= n < 2^31).
+__device__ __forceinline__ int fdiv(int n, FastDiv f) {
+  return (int)(((uint64_t)(uint32_t)n * f.mul) >> f.shift);
+}
+
 struct ChunkMeta {
   int64_t phys;
   int r0;
@@ -99,7 +104,7 @@ struct ChunkMeta {
 __device__ __forceinline__ ChunkMeta chunk_meta(const DecodeArgs& a, int b, int T, int cpp,
                                                 int c) {
   ChunkMeta m;
-  const int lp = c / cpp;
+  const int lp = fdiv(c, a.div_cpp);
   const int j = c - lp * cpp;
   int rows;
   if (a.page_lens) {
@@ -111,7 +116,7 @@ __device__ __forceinline__ ChunkMeta chunk_meta(const DecodeArgs& a, int b, int 
   m.nval = min(16, rows - m.r0);
   const int pg = a.page_table ? ld_ro(a.page_table, (int64_t)b * a.pt_b + lp) : lp;
   m.phys = (int64_t)min(max(pg, 0), a.num_pages - 1);
-  m.group = lp / a.pages_per_group;
+  m.group = fdiv(lp, a.div_ppg);
   m.tok0 = lp * a.page_rows + m.r0;
   return m;
 }
@@ -138,7 +143,8 @@ __device__ __forceinline__ void hand_back_length(const DecodeArgs& a, int b) {
 
 // Logical pages holding the first T rows (T <= max_pages * page_rows).
 __device__ __forceinline__ int pages_of(const DecodeArgs& a, int T) {
-  return T / a.page_rows + (T % a.page_rows != 0);
+  const int full = fdiv(T, a.div_rows);
+  return full + (T != full * a.page_rows);
 }
 
 // Chunks of wave w of `waves` (4 or 8) over the chunks [begin, end) of a

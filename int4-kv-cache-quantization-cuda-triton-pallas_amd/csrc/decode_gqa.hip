@@ -23,6 +23,9 @@
 //      HG probabilities per row, HG float32 FMAs per value element.
 //   The next chunk's loads are in flight while the current one is computed
 //   (two-buffer ping-pong, wait counts exact as in decode_kernel).
+//
+// The planner picks decode_mfma_kernel for grouped heads; this kernel runs under
+// the FDI4_TUNE_DECODE_VECTOR_ONLY override, as its float64 check on the device.
 
 #include "decode_common.hpp"
 
@@ -74,7 +77,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_gqa_kernel(DecodeArgs a) {
 
   const int split = blockIdx.x, b = blockIdx.z;
   const int h0 = blockIdx.y * HG;           // first q-head of this workgroup
-  const int hk = h0 / a.hq_per_kv;          // HG divides hq_per_kv: one kv-head
+  const int hk = fdiv(h0, a.div_hpk);         // HG divides hq_per_kv: one kv-head
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kq = lane % G::LPT;             // channel slice of this lane (K)

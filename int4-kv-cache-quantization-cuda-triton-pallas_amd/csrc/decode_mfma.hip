@@ -1,95 +1,215 @@
-// Fused INT4 flash decoding with the key products on the int8 matrix cores
-// (gfx950, D = 64 or 128). Same semantics as decode_kernel and
-// decode_gqa_kernel (reference src/flash_decode_ref.py:30-139 per (sequence,
-// q-head) stream, q-head h reading kv-head h // (Hq/Hkv), src/ops.py:189-192):
-// unscaled logits sum_d (q_d*s_d)*nib_d - sum_d q_d*(zp_d*s_d), online softmax,
-// float32 value accumulation, split partials or the final output. One
-// workgroup serves HG (2, 4 or 8) q-heads of one kv-head.
+// Fused INT4 flash decoding for grouped query heads on the matrix cores
+// (gfx950): key products on the int8 ones, value products on the 16-bit (16-bit
+// values) or float32 ones. Same semantics as decode_kernel and decode_gqa_kernel
+// (reference src/flash_decode_ref.py:30-139 per (sequence, q-head) stream,
+// q-head h reading kv-head h // (Hq/Hkv), src/ops.py:189-192): unscaled logits
+// sum_d (q_d*s_d)*nib_d - sum_d q_d*(zp_d*s_d), online softmax, float32 value
+// accumulation, split partials or the final output. One workgroup serves HG
+// (2, 4 or 8) q-heads of one kv-head.
 //
-// Logits, exactly: per head m and scale group, the products q_d*s_d (exact
-// in double) are scaled by 2^(41-E_m), E_m the binary exponent of the head's
-// largest |q_d*s_d|, and rounded to integers v_d, |v_d| <= 2^41, written as
-// six 7-bit digits v = d0*2^35 + d1*2^28 + ... + d5 (d0 signed, d1..d5 in
-// 0..127: all int8). One v_mfma_i32_16x16x64_i8 per digit and 64 channels
-// multiplies the 16 key rows' nibbles (A, 16 x 64) by the digits of up to 16
-// heads (B, 64 x 16) with exact int32 sums; the six sums recombine exactly in
-// double as (P0*2^28 + P1*2^14 + P2) * 2^(E_m-41), P0 = acc0*128 + acc1 etc.
-// The only rounding is v_d's: |error| <= 2^(E_m-42) per product, below 1e-9
-// of the largest |q_d*s_d| summed over D=128 channels and nibbles <= 15.
+// Lane l: g = l / 16, n = l % 16, head n / CPH, column c = n % CPH of its head
+// (CPH = 16 / HG columns per head). A 16-row chunk goes through a wave as
 //
-// Lane roles (lane l, g = l / 16): A rows are key rows n = l % 16, each lane
-// holding its row's channels of group g (D/8 packed bytes, one 16- or 8-byte
-// load); B columns are heads m = l % 16 with the same channels; the result
-// lane holds rows 4g .. 4g+3 of head m, so the softmax of head m runs across
-// the four lanes l % 16 == m. Probabilities and rescale factors go through
-// LDS to the value lanes, whose loads and float32 FMAs are those of
-// decode_gqa_kernel. Loads are pipelined as in decode_kernel (two buffers,
-// exact wait counts).
+//   logits: the products v_d = q_d*s_d (exact in double) are scaled by
+//      2^(46-E), E the binary exponent of the head's largest, rounded to
+//      integers |v_d| <= 2^46 and written as six balanced base-256 digits (the
+//      bytes of v + 0x808080808080, each less 128). v_mfma_i32_16x16x64_i8
+//      multiplies the 16 rows' nibbles (A: row n, channels of group g) by
+//      digits (B), and the columns of a head hold DIFFERENT digits: all six in
+//      one product at HG = 2, in two at HG = 4, in three at HG = 8. The exact
+//      int32 sums of a row's digits, which lie in neighbouring lanes, meet by
+//      quad permutes (a reduce-scatter over the columns), so each logit is
+//      recombined in double and exponentiated in one lane (two lanes at
+//      HG = 2), not in every column: lane (g, head, c) ends with row
+//      4g + c % 4 (HG = 8: rows 4g + c and 4g + c + 2). Error against double
+//      products: 2^(E-47) per product and the double rounding of the sum.
+//   probabilities: the lane group g that holds the logits of rows 4g .. 4g+3 is
+//      the one that must supply them as the value product's B operand, so they
+//      move by quad permutes too and nothing goes through LDS.
+//   values, 16-bit: lane (g, n) loads its 8 (4 at D = 64) channels of rows
+//      4g .. 4g+3; byte permutes pair the rows, and each 16x16x16 product adds
+//      four rows a lane group to the output of 16 channels x 16 columns. A
+//      float32 probability is the exact sum of three 8-bit (bfloat16) or
+//      11-bit (float16, scaled by 2^15) terms, which sit in different columns
+//      of the head (HG = 8: in the two halves of a 16x16x32 product), so the
+//      products are exact, their sums are float32, and one instruction does all
+//      terms. Only the final output adds the columns up.
+//      A non-finite value times an empty term is NaN where the float32 product
+//      is infinite: a wave that ends with a NaN runs its range again with the
+//      float32 products below.
+//   values, float32: v_mfma_f32_16x16x4_f32, a row of each lane group at a time.
+//      Chunk sums come first and are then added to the rescaled accumulators.
+//
+// What bounds it, and why this form: a chunk of 16-bit values at D = 128 is 5 KB,
+// 0.66 us of a SIMD's share of HBM; float32 FMAs of every value with every
+// head's probability, widening, the LDS round trip of the probabilities and one
+// logit recombination per (row, column) cost more vector-unit time than that at
+// HG = 4 and twice as much at HG = 8. Measured against that form, per call with
+// the merge: B8 Hkv8 Hq32 T8192 bfloat16 37.6 -> 32.6 us (172 MB; the stream
+// itself now runs at 6.8 TB/s, the rest is the first 6 us and the last 3 of a
+// workgroup); D = 256 B4 Hkv4 Hq16 T4095 30.1 -> 19.9 us (against the vector
+// kernel); a B16 Hkv8 Hq64 float16 step of ragged lengths to 4096 56.8 -> 37.6 us;
+// B8 H32 over one float32 stream of 2048 rows 16.0 -> 13.9 us.
 
 #include "decode_common.hpp"
 
 namespace fdi4 {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
-template <int D, int VDT>
+template <int D, int VDT, int HG>
 struct MfmaGeo {
   static constexpr int NB = D / 64;                // 64-channel MFMA blocks
   static constexpr int KW = D / 32;                // packed key words per lane per row
+  static constexpr int CPH = 16 / HG;              // result columns per head
+  static constexpr int NSET = CPH >= 8 ? 1 : CPH == 4 ? 2 : 3;  // digit products per block
+  static constexpr int RN = CPH >= 4 ? 1 : 2;      // logits a lane ends with
+  static constexpr int PPL = HG * D / 64;          // channels of q*s a lane turns into digits
   static constexpr int VEB = VDT == kVF32 ? 4 : 2; // bytes per value element
-  static constexpr int VCL = 16 / VEB;             // value channels per lane
-  static constexpr int VPR = D / VCL;              // lanes per value row
-  static constexpr int RPL = 64 / VPR;             // value rows per sweep
-  static constexpr int VLD = 16 / RPL;             // value sweeps per chunk
+  static constexpr int PB = D * VEB / 16 < 16 ? D * VEB / 16 : 16;  // bytes per value load
+  static constexpr int NP = D * VEB / (16 * PB);   // value loads per lane per row
+  static constexpr int CPP = PB / VEB;             // channels per value load
+  static constexpr int NA = D / 16;                // 16-channel output tiles
   static constexpr int SZI = D / 2;                // 16-byte items in a scale+zp block
   static constexpr int SZL = (SZI + 63) / 64;      // scale+zp loads per lane
   static constexpr int DIGITS = 6;
-  static_assert(D == 64 || D == 128, "int8 MFMA decode: D = 64 or 128");
+  // LDS per wave: the staged scale/zero-point block and the digits of a group
+  // while the wave streams, its partial output afterwards.
+  static constexpr int kDigBytes = DIGITS * HG * D;
+  static constexpr int kStreamBytes = kDigBytes + 16 * D;
+  static constexpr int kAccBytes = 4 * HG * D;
+  static constexpr int kWaveBytes = kStreamBytes > kAccBytes ? kStreamBytes : kAccBytes;
+  static_assert(D == 64 || D == 128 || D == 256, "head_dim");
+  static_assert(HG == 2 || HG == 4 || HG == 8, "heads per workgroup");
 };
 
-// Channel layout of the MFMA operands: lane group g (lanes 16g .. 16g+15)
-// holds the 16-channel piece kb of channels base = 16g (D = 64) or 32g + 16kb
-// (D = 128); slot j (byte j of the B operand) is channel base + 2j for
-// j < 8 (the low nibbles of the packed bytes) and base + 2(j-8) + 1 for
-// j >= 8 (the high nibbles), matching the A operand built from the packed
-// key words.
+// Position of channel d in the operands' order: lane group g holds channels
+// [g*D/4, (g+1)*D/4) in 16-channel blocks, of each block the even channels
+// (low nibbles of the packed bytes) before the odd ones (high nibbles).
+__device__ __forceinline__ int slot_of(int d) {
+  return (d & ~15) | ((d & 1) << 3) | ((d & 15) >> 1);
+}
 
-template <int HG>
-struct HeadF {
-  float v[HG];
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp(unsigned x) {
+  return (unsigned)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xF, 0xF, false);
+}
+
+// Value of lane ^ 4: mirrored within 8 lanes, then within 4.
+__device__ __forceinline__ double xchg4_dpp(double x) {
+  DU v;
+  v.d = x;
+  v.u[0] = dpp<0x1B>(dpp<0x141>(v.u[0]));
+  v.u[1] = dpp<0x1B>(dpp<0x141>(v.u[1]));
+  return v.d;
+}
+
+template <int LO, int HI>
+__device__ __forceinline__ unsigned allreduce_max_u(unsigned x) {
+  if constexpr (LO <= 1 && 1 < HI) x = max(x, xchg_u32<1>(x));
+  if constexpr (LO <= 2 && 2 < HI) x = max(x, xchg_u32<2>(x));
+  if constexpr (LO <= 4 && 4 < HI) x = max(x, xchg_u32<4>(x));
+  if constexpr (LO <= 8 && 8 < HI) x = max(x, xchg_u32<8>(x));
+  if constexpr (LO <= 16 && 16 < HI) x = max(x, xchg_u32<16>(x));
+  if constexpr (LO <= 32 && 32 < HI) x = max(x, xchg_u32<32>(x));
+  return x;
+}
+
+// The chunk walk of a wave: logical page, chunk within it, scale group and the
+// page's index in its group, advanced by compares.
+struct ChunkPos {
+  int lp, j, group, pig;
 };
+
+__device__ __forceinline__ ChunkPos chunk_pos(const DecodeArgs& a, int c, int cpp) {
+  ChunkPos p;
+  p.lp = fdiv(c, a.div_cpp);
+  p.j = c - p.lp * cpp;
+  p.group = fdiv(p.lp, a.div_ppg);
+  p.pig = p.lp - p.group * a.pages_per_group;
+  return p;
+}
+
+__device__ __forceinline__ ChunkPos chunk_next(ChunkPos p, int cpp, int ppg) {
+  p.j += 1;
+  const bool np = p.j == cpp;
+  p.j = np ? 0 : p.j;
+  p.lp += np ? 1 : 0;
+  p.pig += np ? 1 : 0;
+  const bool ng = p.pig == ppg;
+  p.pig = ng ? 0 : p.pig;
+  p.group += ng ? 1 : 0;
+  return p;
+}
+
+struct PosMeta {
+  int64_t phys;
+  int r0, nval, group;
+};
+
+__device__ __forceinline__ PosMeta pos_meta(const DecodeArgs& a, int b, int T,
+                                            const ChunkPos& p) {
+  PosMeta m;
+  int rows;
+  if (a.page_lens) {
+    rows = min(max(ld_ro(a.page_lens, (int64_t)b * a.pl_b + p.lp), 0), a.page_rows);
+  } else {
+    rows = min(a.page_rows, T - p.lp * a.page_rows);
+  }
+  m.r0 = p.j * 16;
+  m.nval = min(16, rows - m.r0);
+  const int pg = a.page_table ? ld_ro(a.page_table, (int64_t)b * a.pt_b + p.lp) : p.lp;
+  m.phys = (int64_t)min(max(pg, 0), a.num_pages - 1);
+  m.group = p.group;
+  return m;
+}
 
 template <int D, int VDT, int WAVES, int HG>
 __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
-  using G = MfmaGeo<D, VDT>;
-  constexpr int NT = WAVES * 64;
-  static_assert(HG >= 2 && HG <= 8, "heads per workgroup");
+  using G = MfmaGeo<D, VDT, HG>;
+  constexpr int NT = WAVES * 64, CPH = G::CPH, RN = G::RN;
+  // float16 terms of a probability are those of p * 2^15 (still finite), so
+  // that they keep 24 bits down to p = 2^-15 and 2^-39 below.
+  constexpr float kPScale = VDT == kVF16 ? 32768.f : 1.f;
 
   const int split = blockIdx.x, b = blockIdx.z;
   const int h0 = blockIdx.y * HG;           // first q-head of this workgroup
-  const int hk = h0 / a.hq_per_kv;          // HG divides hq_per_kv: one kv-head
+  const int hk = fdiv(h0, a.div_hpk);         // HG divides hq_per_kv: one kv-head
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n16 = lane & 15;                // key row (A) and head (B, result)
+  const int n16 = lane & 15;                // key row (A) and result column
   const int grp = lane >> 4;                // channel group; result rows 4*grp..+3
-  const bool head_lane = n16 < HG;
-  const int vrow = lane / G::VPR;
-  const int vcol = lane % G::VPR;
+  const int hh = n16 / CPH;                 // head of this lane's column
+  const int col = n16 % CPH;                // column within the head
+  const bool odd = (n16 & 1) != 0, hi2 = (n16 & 2) != 0, hi4 = (n16 & 4) != 0;
+  const int lrow = 4 * grp + (CPH >= 4 ? (n16 & 3) : (n16 & 1));  // row of logit 0
 
-  __shared__ float q_s[HG][D];
-  __shared__ HeadF<HG> p_s[WAVES][16];
-  __shared__ HeadF<HG> corr_s[WAVES];
-  __shared__ float sz_s[WAVES][2 * D];
-  __shared__ float acc_s[WAVES][HG][D];
+  __shared__ __align__(16) float q_s[HG][D];                      // slot order
+  __shared__ __align__(16) uint8_t wave_s[WAVES][G::kWaveBytes];
   __shared__ double m_s[WAVES][HG];
   __shared__ float l_s[WAVES][HG];
-  // Per wave: the HG heads' B operands in MFMA lane layout [digit][block]
-  // [channel group][head][byte], their exponents and group constants.
-  __shared__ __attribute__((aligned(16))) uint8_t dig_s[WAVES][G::DIGITS][G::NB][4][HG][16];
-  __shared__ int hex_s[WAVES][HG];
-  __shared__ double hcg_s[WAVES][HG];
+  uint8_t* const dig_w = wave_s[w];
+  double* const sz_w = reinterpret_cast<double*>(wave_s[w] + G::kDigBytes);
 
-  const int cpp = (a.page_rows + 15) >> 4;
+  // The q rows of the HG heads are loaded first and go to LDS once the first
+  // chunk's loads are issued.
+  constexpr int QPT = (HG * D + NT - 1) / NT;
+  float qv[QPT];
+#pragma unroll
+  for (int j = 0; j < QPT; ++j) {
+    const int idx = tid + j * NT;
+    qv[j] = (idx < HG * D)
+                ? load_elem(a.q, (int64_t)b * a.q_b + (int64_t)(h0 + idx / D) * a.q_h + idx % D,
+                            a.q_dtype)
+                : 0.f;
+  }
+
+  const int cpp = (a.page_rows + 15) >> 4, ppg = a.pages_per_group;
   const int T = seq_len_of(a, b);
   const int n_chunks = pages_of(a, T) * cpp;
   const int c_begin = split * a.chunks_per_split;
@@ -97,19 +217,15 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   const WaveRange wr = wave_chunks(c_begin, c_end, w, WAVES);
   const int wc0 = wr.c0, wc1 = wr.c1;
 
-  // Softmax state of head n16 (meaningful on head lanes).
+  // Softmax state of head hh in units of log2 (the same in all its lanes), and
+  // the sum of the probabilities of this lane's rows.
   double m_run = -INFINITY;
   float l_run = 0.f;
-  double cg = 0.0;
-  int e_head = 0;
-  // Value accumulators of all HG heads for this lane's value channels.
-  float acc[HG][G::VCL];
-#pragma unroll
-  for (int h = 0; h < HG; ++h)
-#pragma unroll
-    for (int k = 0; k < G::VCL; ++k) acc[h][k] = 0.f;
-  // Digits of head n16's scaled q*s for this lane's channels (B operands).
-  v4i bq[G::DIGITS][G::NB];
+  // Output tiles: channel 8 (CPP) * m + j of piece u for result row m, column n16.
+  v4f acc[G::NA];
+  // Digits of head hh's scaled q*s (B operands), and logit = sum * c1 - cg.
+  v4i bq[G::NSET][G::NB];
+  double c1 = 0.0, cg = 0.0;
   int cur_group = -1;
 
   const float* sbase = a.k_scale + (int64_t)b * a.s_b + (int64_t)hk * a.s_h;
@@ -121,10 +237,15 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   const uint8_t* kbase_h = a.k_pages + (int64_t)hk * a.k_head;
   const uint8_t* vbase_h = reinterpret_cast<const uint8_t*>(a.v_pages) +
                            (int64_t)hk * a.v_head * G::VEB;
-  const unsigned k_lane = grp * (D / 8), v_lane = vcol * 16;
+  const unsigned k_lane = grp * (D / 8), v_lane = n16 * G::PB;
   const unsigned krow_b = (unsigned)a.k_row, vrow_b = (unsigned)(a.v_row * G::VEB);
 
-  auto load_sz = [&](const ChunkMeta& m, U32x4* sz) {
+  struct Buf {
+    unsigned k[G::KW];
+    unsigned v[4][G::NP][G::PB / 4];
+  };
+
+  auto load_sz = [&](const PosMeta& m, U32x4* sz) __attribute__((always_inline)) {
     const int64_t off = (int64_t)m.group * a.s_g + m.phys * a.s_p;
 #pragma unroll
     for (int i = 0; i < G::SZL; ++i) {
@@ -134,257 +255,491 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     }
   };
 
-  auto load_chunk = [&](const ChunkMeta& m, KVec<G::KW>* kr, U32x4* vr) {
+  // Rows past the valid count are loaded from the last valid row (never out of
+  // bounds); their probabilities are 0.
+  auto load_chunk = [&](const PosMeta& m, int nval, Buf& f) __attribute__((always_inline)) {
     const uint8_t* kb = kbase_h + m.phys * a.k_page + (int64_t)m.r0 * a.k_row;
-    const int t = max(min(n16, m.nval - 1), 0);
-    kr[0] = load_k<G::KW>(kb + (k_lane + (unsigned)t * krow_b));
+    const unsigned ko = k_lane + (unsigned)max(min(n16, nval - 1), 0) * krow_b;
+    constexpr int KL = G::KW < 4 ? G::KW : 4;
+#pragma unroll
+    for (int i = 0; i < G::KW / KL; ++i) {
+      const KVec<KL> x = load_k<KL>(kb + (ko + 16 * i));
+#pragma unroll
+      for (int k = 0; k < KL; ++k) f.k[KL * i + k] = x.w[k];
+    }
     const uint8_t* vb = vbase_h + (m.phys * a.v_page + (int64_t)m.r0 * a.v_row) * G::VEB;
 #pragma unroll
-    for (int i = 0; i < G::VLD; ++i) {
-      const int r = max(min(i * G::RPL + vrow, m.nval - 1), 0);
-      vr[i] = ld16_stream(vb + (v_lane + (unsigned)r * vrow_b));
+    for (int i = 0; i < 4; ++i) {
+      const unsigned vo = v_lane + (unsigned)max(min(4 * grp + i, nval - 1), 0) * vrow_b;
+#pragma unroll
+      for (int u = 0; u < G::NP; ++u) {
+        const KVec<G::PB / 4> x = load_k<G::PB / 4>(vb + (vo + 16 * G::PB * u));
+#pragma unroll
+        for (int k = 0; k < G::PB / 4; ++k) f.v[i][u][k] = x.w[k];
+      }
     }
   };
 
-  // Rebuild the B operands (digits), exponents and group constants of the HG
-  // heads from the staged scale/zero-point block. The products are spread
-  // densely: lane l computes PPL channels of head l / LPH (every lane busy,
-  // whatever HG), and the digit bytes go through LDS into the MFMA lane
-  // layout (lane l's B operand: head l % 16, channel group l / 16), where a
-  // head lane reads them back as 16-byte words.
-  auto rebuild = [&](const float* szw) {
-    constexpr int LPH = 64 / HG;        // lanes per head
-    constexpr int PPL = HG * D / 64;    // channels per lane
-    const int hh = lane / LPH;
-    const int d0 = (lane % LPH) * PPL;
-    const float* qh = q_s[hh];
-    // Pass 1: the head's largest |q*s| (its exponent) and the group constant.
-    double mx = 0.0, cgp = 0.0;
+  // Rebuild the B operands (digits), scale factors and group constants of the
+  // HG heads from the loaded scale/zero-point block. Lane (g, head, c) turns
+  // the PPL channels at slots c*PPL of its group into digits; the bytes go
+  // through LDS ([digit][head][slot]) to the lanes whose column needs them.
+  auto rebuild = [&](const U32x4* sz) __attribute__((always_inline)) {
+    // Staged as doubles, in slot order: the conversions are shared by the heads.
 #pragma unroll
-    for (int i = 0; i < PPL; ++i) {
-      const int d = d0 + i;
-      const double qd = (double)qh[d];
-      const double sd = (double)szw[d];
-      mx = fmax(mx, fabs(qd * sd));
-      cgp = __builtin_fma(qd, (double)szw[D + d] * sd, cgp);
-    }
-    mx = allreduce_max<1, LPH>(mx);
-    const double cgh = allreduce_sum<1, LPH>(cgp);
-    int ex = 0;
-    if (mx > 0.0) (void)frexp(mx, &ex);
-    // Pass 2: the products again (cheaper than keeping them), as digits at
-    // their B-operand byte: channel d is byte j of group g's block kb.
-#pragma unroll
-    for (int i = 0; i < PPL; ++i) {
-      const int d = d0 + i;
-      const double qsd = (double)qh[d] * (double)szw[d];
-      // v = rint(q*s * 2^(41 - e)), |v| <= 2^41; v = hi * 2^21 + lo, 0 <= lo < 2^21.
-      const double v = rint(ldexp(qsd, 41 - ex));
-      const double hi = floor(v * 0x1p-21);
-      const int hi_i = (int)hi;
-      const int lo_i = (int)(v - hi * 0x1p21);
-      const unsigned dig[G::DIGITS] = {
-          (unsigned)(hi_i >> 14) & 255u, (unsigned)(hi_i >> 7) & 127u, (unsigned)hi_i & 127u,
-          (unsigned)(lo_i >> 14) & 127u, (unsigned)(lo_i >> 7) & 127u, (unsigned)lo_i & 127u};
-      const int g = (D == 64) ? d / 16 : d / 32;
-      const int kb = (D == 64) ? 0 : (d / 16) & 1;
-      const int o = d & 15;
-      const int jb = (o & 1) ? 8 + (o >> 1) : (o >> 1);
-#pragma unroll
-      for (int dg = 0; dg < G::DIGITS; ++dg) dig_s[w][dg][kb][g][hh][jb] = (uint8_t)dig[dg];
-    }
-    if (lane % LPH == 0) {
-      hex_s[w][hh] = ex;
-      hcg_s[w][hh] = cgh;
+    for (int i = 0; i < G::SZL; ++i) {
+      const int e = i * 64 + lane;
+      if (e < G::SZI) {
+        double* dst = sz_w + (e < D / 4 ? 0 : D) + slot_of(4 * (e % (D / 4)));
+        *reinterpret_cast<double2*>(dst) = make_double2(u2f(sz[i].x), u2f(sz[i].z));
+        *reinterpret_cast<double2*>(dst + 8) = make_double2(u2f(sz[i].y), u2f(sz[i].w));
+      }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (head_lane) {
+    constexpr int PPL = G::PPL, PK = PPL < 4 ? PPL : 4;
+    const int s0 = grp * (D / 4) + col * PPL;
+    const float* qh = q_s[hh] + s0;
+    const double* sh = sz_w + s0;
+    const double* zh = sz_w + D + s0;
+    // The largest |q*s| by its high word (exponent and leading bits), and the
+    // group constant.
+    unsigned mx = 0;
+    double cgp = 0.0;
+    DU qs[PPL];
 #pragma unroll
-      for (int dg = 0; dg < G::DIGITS; ++dg)
+    for (int i = 0; i < PPL; ++i) {
+      const double qd = (double)qh[i], sd = sh[i];
+      qs[i].d = qd * sd;
+      mx = max(mx, qs[i].u[1] & 0x7FFFFFFFu);
+      cgp = __builtin_fma(qd, zh[i] * sd, cgp);
+    }
+    mx = allreduce_max_u<16, 64>(allreduce_max_u<1, CPH>(mx));
+    cgp = allreduce_sum<16, 64>(allreduce_sum<1, CPH>(cgp));
+    // |q*s| < 2^E, E = (mx >> 20) - 1022; all zero, infinite or NaN (then the
+    // group constant is too): any scale.
+    const int E = mx - 1u < 0x7FEFFFFFu ? (int)(mx >> 20) - 1022 : 0;
+    DU up, down;
+    up.u[0] = 0;
+    up.u[1] = (unsigned)(1023 + 46 - E) << 20;
+    down.u[0] = 0;
+    down.u[1] = (unsigned)(1023 - 46 + E) << 20;
+    c1 = down.d * 1.4426950408889634;
+    cg = cgp * 1.4426950408889634;
+    // 1.5 * 2^52 + the bias of the balanced digits: the low 48 bits of the sum
+    // are rint(q*s * 2^(46-E)) + 0x808080808080.
+    constexpr double kMagic = 6755399441055744.0 + 141289400074368.0;
 #pragma unroll
-        for (int kb = 0; kb < G::NB; ++kb)
-          bq[dg][kb] = *reinterpret_cast<const v4i*>(&dig_s[w][dg][kb][grp][n16][0]);
-      e_head = hex_s[w][n16];
-      cg = hcg_s[w][n16];
+    for (int i0 = 0; i0 < PPL; i0 += PK) {
+      unsigned lo[4] = {0, 0, 0, 0}, hi[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < PK; ++k) {
+        DU v;
+        v.d = __builtin_fma(qs[i0 + k].d, up.d, kMagic);
+        lo[k] = v.u[0];
+        hi[k] = v.u[1];
+      }
+      const unsigned t0 = __builtin_amdgcn_perm(lo[1], lo[0], 0x05010400u);
+      const unsigned t1 = __builtin_amdgcn_perm(lo[1], lo[0], 0x07030602u);
+      const unsigned u0 = __builtin_amdgcn_perm(lo[3], lo[2], 0x05010400u);
+      const unsigned u1 = __builtin_amdgcn_perm(lo[3], lo[2], 0x07030602u);
+      const unsigned h0w = __builtin_amdgcn_perm(hi[1], hi[0], 0x05010400u);
+      const unsigned h1w = __builtin_amdgcn_perm(hi[3], hi[2], 0x05010400u);
+      // Digit 0 is the most significant.
+      const unsigned dg[6] = {
+          __builtin_amdgcn_perm(h1w, h0w, 0x07060302u), __builtin_amdgcn_perm(h1w, h0w, 0x05040100u),
+          __builtin_amdgcn_perm(u1, t1, 0x07060302u),   __builtin_amdgcn_perm(u1, t1, 0x05040100u),
+          __builtin_amdgcn_perm(u0, t0, 0x07060302u),   __builtin_amdgcn_perm(u0, t0, 0x05040100u)};
+#pragma unroll
+      for (int k = 0; k < G::DIGITS; ++k) {
+        uint8_t* dst = dig_w + k * HG * D + hh * D + s0 + i0;
+        if constexpr (PK == 4)
+          *reinterpret_cast<unsigned*>(dst) = dg[k] ^ 0x80808080u;
+        else
+          *reinterpret_cast<uint16_t*>(dst) = (uint16_t)(dg[k] ^ 0x8080u);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int s = 0; s < G::NSET; ++s) {
+      // The digit of this lane's column in product s.
+      int dg;
+      if constexpr (CPH == 2) dg = 2 * s + col;
+      else if constexpr (CPH == 4) dg = s == 0 ? col : 4 + (col & 1);
+      else dg = hi4 ? 4 + (col & 1) : (col & 3);
+#pragma unroll
+      for (int kb = 0; kb < G::NB; ++kb)
+        bq[s][kb] = *reinterpret_cast<const v4i*>(dig_w + dg * HG * D + hh * D +
+                                                  grp * (D / 4) + 16 * kb);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  // Column sums of a digit pair: lane pairs (even column: high digit) exchange
+  // rows, the even lane keeping rows 0 and 2 of its four, the odd one 1 and 3.
+  const int wsh = odd ? 0 : 8;
+  auto pair_rows = [&](const v4i& d, int* r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int keep = (odd ? d[2 * k + 1] : d[2 * k]) << wsh;
+      const int send = (odd ? d[2 * k] : d[2 * k + 1]) << wsh;
+      r[k] = keep + (int)dpp<0xB1>((unsigned)send);
+    }
+  };
+  // Weights of the lane's own digit pair and of the pair its partner sends.
+  const double w_own = CPH >= 8 && hi4 ? 1.0 : hi2 ? 0x1p16 : 0x1p32;
+  const double w_oth = CPH >= 8 && hi4 ? 0.0 : hi2 ? 0x1p32 : 0x1p16;
+
+  // Logits (log2 units) of the lane's RN rows.
+  auto logits = [&](const Buf& f, double* lg) __attribute__((always_inline)) {
+    v4i ds[G::NSET];
+#pragma unroll
+    for (int kb = 0; kb < G::NB; ++kb) {
+      const unsigned w0 = f.k[2 * kb], w1 = f.k[2 * kb + 1];
+      const v4i ak = v4i{(int)(w0 & 0x0F0F0F0Fu), (int)(w1 & 0x0F0F0F0Fu),
+                         (int)((w0 >> 4) & 0x0F0F0F0Fu), (int)((w1 >> 4) & 0x0F0F0F0Fu)};
+#pragma unroll
+      for (int s = 0; s < G::NSET; ++s)
+        ds[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak, bq[s][kb],
+                                                      kb == 0 ? v4i{0, 0, 0, 0} : ds[s], 0, 0, 0);
+    }
+    if constexpr (CPH == 2) {
+      int p[3][2];
+#pragma unroll
+      for (int s = 0; s < 3; ++s) pair_rows(ds[s], p[s]);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const double s = __builtin_fma((double)p[0][k], 0x1p32,
+                                       __builtin_fma((double)p[1][k], 0x1p16, (double)p[2][k]));
+        lg[k] = __builtin_fma(s, c1, -cg);
+      }
     } else {
-#pragma unroll
-      for (int dg = 0; dg < G::DIGITS; ++dg)
-#pragma unroll
-        for (int kb = 0; kb < G::NB; ++kb) bq[dg][kb] = v4i{0, 0, 0, 0};
-      e_head = 0;
-      cg = 0.0;
+      int p[2];
+      pair_rows(ds[0], p);
+      const int own = hi2 ? p[1] : p[0];
+      const int oth = (int)dpp<0x4E>((unsigned)(hi2 ? p[0] : p[1]));
+      double s;
+      if constexpr (CPH == 4) {
+        int r[2];
+        pair_rows(ds[1], r);
+        s = __builtin_fma((double)own, w_own,
+                          __builtin_fma((double)oth, w_oth, (double)(hi2 ? r[1] : r[0])));
+      } else {
+        s = __builtin_fma((double)own, w_own, (double)oth * w_oth);
+        s += xchg4_dpp(s);
+      }
+      lg[0] = __builtin_fma(s, c1, -cg);
     }
   };
 
+  // Float32 products of the values with the four rows' probabilities x, added
+  // to the accumulators rescaled by corr. A chunk's rows are summed by
+  // themselves first, in two chains of eight: one rounding per chunk reaches
+  // the running sum, not one per row (measured against one chain through all
+  // rows: 2.3e-7 -> 1.9e-7 of the result at T 15000).
+  auto value_f32 = [&](const Buf& f, const float* x, float corr) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < G::NP; ++u)
+#pragma unroll
+      for (int j = 0; j < G::CPP; ++j) {
+        v4f t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v;
+          if constexpr (VDT == kVF32) v = u2f(f.v[i][u][j]);
+          else if constexpr (VDT == kVF16)
+            v = (float)__builtin_bit_cast(_Float16,
+                                          (unsigned short)(f.v[i][u][j / 2] >> (16 * (j & 1))));
+          else v = u2f(j & 1 ? f.v[i][u][j / 2] & 0xFFFF0000u : f.v[i][u][j / 2] << 16);
+          t[i / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, x[i], t[i / 2], 0, 0, 0);
+        }
+        v4f& o = acc[u * G::CPP + j];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(o[i], corr, t[0][i] + t[1][i]);
+      }
+  };
+
+  // Upper bits of a probability that one 16-bit term holds.
+  constexpr unsigned kTerm = VDT == kVF16 ? 0xFFFFE000u : 0xFFFF0000u;
+  // Two terms packed as the 16-bit type (their lower bits are zero or, below
+  // the smallest, dropped).
+  auto pack2 = [&](float lo, float hi) __attribute__((always_inline)) -> unsigned {
+    if constexpr (VDT == kVF16)
+      return __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+    else
+      return __builtin_amdgcn_perm(f2u(hi), f2u(lo), 0x07060302u);
+  };
+  const unsigned term1 = col >= 1 ? kTerm : 0u, term2 = col >= 2 ? kTerm : 0u;
+
+  // 16-bit products of the values with the terms of the probabilities x.
+  auto value_16 = [&](const Buf& f, const float* x) __attribute__((always_inline)) {
+    unsigned bt[4];
+    if constexpr (CPH == 2) {
+      // Column 0: first and second term; column 1: third term and nothing.
+      float ta[4], tb[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float r1 = x[i] - u2f(f2u(x[i]) & kTerm);
+        const float r2 = r1 - u2f(f2u(r1) & kTerm);
+        ta[i] = odd ? r2 : x[i];
+        tb[i] = odd ? 0.f : r1;
+      }
+      bt[0] = pack2(ta[0], ta[1]);
+      bt[1] = pack2(ta[2], ta[3]);
+      bt[2] = pack2(tb[0], tb[1]);
+      bt[3] = pack2(tb[2], tb[3]);
+    } else {
+      // Column c: term c (columns 3 and beyond repeat term 2 and are dropped).
+      float t[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        t[i] = x[i] - u2f(f2u(x[i]) & term1);
+        t[i] = t[i] - u2f(f2u(t[i]) & term2);
+      }
+      bt[0] = pack2(t[0], t[1]);
+      bt[1] = pack2(t[2], t[3]);
+      bt[2] = bt[3] = 0;
+    }
+#pragma unroll
+    for (int u = 0; u < G::NP; ++u)
+#pragma unroll
+      for (int j = 0; j < G::CPP; ++j) {
+        const unsigned sel = j & 1 ? 0x07060302u : 0x05040100u;
+        const unsigned a0 = __builtin_amdgcn_perm(f.v[1][u][j / 2], f.v[0][u][j / 2], sel);
+        const unsigned a1 = __builtin_amdgcn_perm(f.v[3][u][j / 2], f.v[2][u][j / 2], sel);
+        v4f& t = acc[u * G::CPP + j];
+        if constexpr (CPH == 2) {
+          const U32x4 av = {a0, a1, a0, a1}, bv = {bt[0], bt[1], bt[2], bt[3]};
+          if constexpr (VDT == kVF16)
+            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, av),
+                                                       __builtin_bit_cast(v8h, bv), t, 0, 0, 0);
+          else
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, av),
+                                                        __builtin_bit_cast(v8b, bv), t, 0, 0, 0);
+        } else {
+          const uint2 av = make_uint2(a0, a1), bv = make_uint2(bt[0], bt[1]);
+          if constexpr (VDT == kVF16)
+            t = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, av),
+                                                      __builtin_bit_cast(v4h, bv), t, 0, 0, 0);
+          else
+            t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(v4s, av),
+                                                          __builtin_bit_cast(v4s, bv), t, 0, 0, 0);
+        }
+      }
+  };
+
+  // Consume one chunk of nval > 0 rows. wide: float32 products also for 16-bit
+  // values.
+  auto consume = [&](const Buf& f, int nval, bool wide) __attribute__((always_inline)) {
+    double lg[RN];
+    logits(f, lg);
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < RN; ++k) {
+      lg[k] = lrow + 2 * k < nval ? lg[k] : -INFINITY;
+      mloc = fmaxf(mloc, (float)lg[k]);
+    }
+    float mc = allreduce_max_f<1, (CPH >= 4 ? 4 : 2)>(mloc);
+    mc = allreduce_max_f<16, 64>(mc);
+    // The shift: the float32 maximum of the rounded logits, raised by two of
+    // its ulps so that no probability exceeds 1 -- or, where two ulps are more
+    // than a quarter, the double maximum itself.
+    double mx = __builtin_fma(__builtin_fabs((double)mc), 0x1p-22, (double)mc);
+    if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(mc) < 0x1p20f))) {
+      mx = lg[0];
+      if constexpr (RN > 1) mx = fmax(mx, lg[RN - 1]);
+      mx = allreduce_max<16, 64>(allreduce_max<1, (CPH >= 4 ? 4 : 2)>(mx));
+    }
+    const double m_new = fmax(m_run, mx);
+    const float corr = __builtin_amdgcn_exp2f((float)(m_run - m_new));
+    m_run = m_new;
+    float p[RN], psum = 0.f;
+#pragma unroll
+    for (int k = 0; k < RN; ++k) {
+      p[k] = __builtin_amdgcn_exp2f((float)(lg[k] - m_new)) * kPScale;
+      psum += p[k];
+    }
+    l_run = l_run * corr + psum;
+    // Most chunks do not move the maximum of any head.
+    if (VDT != kVF32 && __builtin_amdgcn_ballot_w64(corr != 1.f)) {
+#pragma unroll
+      for (int t = 0; t < G::NA; ++t) acc[t] *= corr;
+    }
+    float x[4];
+    if constexpr (CPH >= 4) {
+      x[0] = u2f(dpp<0x00>(f2u(p[0])));
+      x[1] = u2f(dpp<0x55>(f2u(p[0])));
+      x[2] = u2f(dpp<0xAA>(f2u(p[0])));
+      x[3] = u2f(dpp<0xFF>(f2u(p[0])));
+    } else {
+      x[0] = u2f(dpp<0xA0>(f2u(p[0])));
+      x[1] = u2f(dpp<0xF5>(f2u(p[0])));
+      x[2] = u2f(dpp<0xA0>(f2u(p[RN - 1])));
+      x[3] = u2f(dpp<0xF5>(f2u(p[RN - 1])));
+    }
+    if constexpr (VDT == kVF32) {
+      value_f32(f, x, corr);
+    } else {
+      if (wide) value_f32(f, x, 1.f);
+      else value_16(f, x);
+    }
+  };
+
+  // One step: (1) rebuild for a new scale group, (2) prefetch chunk c+1 (one row
+  // of the last chunk on the last step, so that every step issues the same loads
+  // and the wait counts stay exact), (3) read the page-table entry of chunk c+2
+  // on the scalar unit, (4) consume chunk c. Called alternately with the two
+  // buffers swapped, so no register copy waits on the prefetch.
   int c = wc0;
-  ChunkMeta cm, nm;
+  ChunkPos np{};
+  PosMeta cm{}, nm{};
   U32x4 sz[G::SZL];
-  auto meta_at = [&](int ci) { return chunk_meta(a, b, T, cpp, min(ci, wc1 - 1)); };
-  auto step = [&](const KVec<G::KW>* ck, const U32x4* cv, KVec<G::KW>* nk, U32x4* nv) -> bool {
+  auto advance = [&](int ci) __attribute__((always_inline)) {
+    if (ci < wc1) np = chunk_next(np, cpp, ppg);
+  };
+  auto step = [&](const Buf& f, Buf& nf) __attribute__((always_inline)) -> bool {
     if (cm.group != cur_group) {
-      float* szw = sz_s[w];
-#pragma unroll
-      for (int i = 0; i < G::SZL; ++i) {
-        const int e = i * 64 + lane;
-        if (e < G::SZI) *reinterpret_cast<U32x4*>(szw + 4 * e) = sz[i];
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      rebuild(szw);
+      rebuild(sz);
       cur_group = cm.group;
-      __builtin_amdgcn_wave_barrier();
     }
-
     const bool last = c + 1 >= wc1;
-    ChunkMeta pf = nm;
-    pf.nval = last ? 1 : nm.nval;
-    load_sz(pf, sz);
-    load_chunk(pf, nk, nv);
-    const ChunkMeta nnm = meta_at(c + 2);
-    if (cm.nval > 0) {
-      // Key rows x digits: acc[dg][r] = sum over channels of nib * digit for
-      // row 4*grp + r of head n16.
-      v4i accd[G::DIGITS];
-#pragma unroll
-      for (int kb = 0; kb < G::NB; ++kb) {
-        const unsigned w0 = ck[0].w[2 * kb], w1 = ck[0].w[2 * kb + 1];
-        const v4i ak = v4i{(int)(w0 & 0x0F0F0F0Fu), (int)(w1 & 0x0F0F0F0Fu),
-                           (int)((w0 >> 4) & 0x0F0F0F0Fu), (int)((w1 >> 4) & 0x0F0F0F0Fu)};
-#pragma unroll
-        for (int dg = 0; dg < G::DIGITS; ++dg)
-          accd[dg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-              ak, bq[dg][kb], kb == 0 ? v4i{0, 0, 0, 0} : accd[dg], 0, 0, 0);
-      }
-      double lg[4];
-      float mloc = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int p0 = accd[0][r] * 128 + accd[1][r];
-        const int p1 = accd[2][r] * 128 + accd[3][r];
-        const int p2 = accd[4][r] * 128 + accd[5][r];
-        const double s = __builtin_fma((double)p0, 0x1p28,
-                                       __builtin_fma((double)p1, 0x1p14, (double)p2));
-        lg[r] = (4 * grp + r < cm.nval) ? ldexp(s, e_head - 41) - cg : -INFINITY;
-        mloc = fmaxf(mloc, (float)lg[r]);
-      }
-      // The float32 maximum of the rounded logits (exact as a double) is the
-      // shift; lg - m_new stays <= half a float ulp of lg.
-      const float mc = allreduce_max_f<16, 64>(mloc);
-      const double m_new = fmax(m_run, (double)mc);
-      const float corr = exp2_of(m_run - m_new);
-      m_run = m_new;
-      float psum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = exp2_of(lg[r] - m_new);
-        psum += p;
-        if (head_lane) p_s[w][4 * grp + r].v[head_lane ? n16 : 0] = p;
-      }
-      l_run = l_run * corr + psum;
-      if (head_lane && grp == 0) corr_s[w].v[head_lane ? n16 : 0] = corr;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-      const HeadF<HG> cr = corr_s[w];
-#pragma unroll
-      for (int h = 0; h < HG; ++h)
-#pragma unroll
-        for (int k = 0; k < G::VCL; ++k) acc[h][k] *= cr.v[h];
-#pragma unroll
-      for (int i = 0; i < G::VLD; ++i) {
-        // Rows past the valid count hold probability 0 and a copy of a valid row.
-        const HeadF<HG> pr = p_s[w][i * G::RPL + vrow];
-        float vf[G::VCL];
-        widen_values<VDT>(cv[i], vf);
-#pragma unroll
-        for (int h = 0; h < HG; ++h)
-#pragma unroll
-          for (int k = 0; k < G::VCL; ++k) acc[h][k] = __builtin_fmaf(pr.v[h], vf[k], acc[h][k]);
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
+    load_sz(nm, sz);
+    load_chunk(nm, last ? 1 : nm.nval, nf);
+    advance(c + 2);
+    const PosMeta nnm = pos_meta(a, b, T, np);
+    if (cm.nval > 0) consume(f, cm.nval, false);
     c += 1;
     cm = nm;
     nm = nnm;
     return last;
   };
 
-  // q rows of the HG heads: into registers first, then the first chunk's
-  // loads, then q to LDS (as in decode_kernel).
-  constexpr int QPT = (HG * D + NT - 1) / NT;
-  float qv[QPT];
-#pragma unroll
-  for (int j = 0; j < QPT; ++j) {
-    const int idx = tid + j * NT;
-    qv[j] = (idx < HG * D)
-                ? load_elem(a.q, (int64_t)b * a.q_b + (int64_t)(h0 + idx / D) * a.q_h + idx % D,
-                            a.q_dtype)
-                : 0.f;
-  }
-  const bool has_work = c < wc1;
-  KVec<G::KW> ka[1], kb[1];
-  U32x4 va[G::VLD], vb[G::VLD];
-  if (has_work) {
-    cm = meta_at(c);
-    nm = meta_at(c + 1);
+  const bool has_work = wc0 < wc1;
+  Buf fa, fb;
+  auto first_loads = [&]() __attribute__((always_inline)) {
+    np = chunk_pos(a, wc0, cpp);
+    cm = pos_meta(a, b, T, np);
+    advance(wc0 + 1);
+    nm = pos_meta(a, b, T, np);
     load_sz(cm, sz);
-    load_chunk(cm, ka, va);
-  }
+    load_chunk(cm, cm.nval, fa);
+  };
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < G::NA; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  };
+  if (has_work) first_loads();
 #pragma unroll
   for (int j = 0; j < QPT; ++j) {
     const int idx = tid + j * NT;
-    if (idx < HG * D) q_s[idx / D][idx % D] = qv[j];
+    if (idx < HG * D) q_s[idx / D][slot_of(idx % D)] = qv[j];
   }
+  clear();
   __syncthreads();
   if (has_work) {
     while (true) {
-      if (step(ka, va, kb, vb)) break;
-      if (step(kb, vb, ka, va)) break;
+      if (step(fa, fb)) break;
+      if (step(fb, fa)) break;
     }
   }
 
-  // Wave totals per head, then the log-sum-exp merge of the waves.
-  const float l_tot = allreduce_sum<16, 64>(l_run);
-  if (head_lane && grp == 0) {
-    m_s[w][head_lane ? n16 : 0] = m_run;
-    l_s[w][head_lane ? n16 : 0] = l_tot;
+  if constexpr (VDT != kVF32) {
+    // Columns beyond the three terms hold nothing.
+    int cols = CPH == 2 ? 2 : 3;
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < G::NA; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bad |= !(acc[t][i] == acc[t][i]);
+    if (__builtin_amdgcn_ballot_w64(bad)) {
+      // Rare (an infinite or NaN value or query): the range again, one chunk at
+      // a time, with float32 products, whose columns are all the full sum.
+      clear();
+      m_run = -INFINITY;
+      l_run = 0.f;
+      cols = 1;
+      ChunkPos p = chunk_pos(a, wc0, cpp);
+      for (int ci = wc0; ci < wc1; ++ci) {
+        const PosMeta m = pos_meta(a, b, T, p);
+        load_sz(m, sz);
+        load_chunk(m, m.nval, fa);
+        if (m.group != cur_group) {
+          rebuild(sz);
+          cur_group = m.group;
+        }
+        if (m.nval > 0) consume(fa, m.nval, true);
+        p = chunk_next(p, cpp, ppg);
+      }
+    }
+    // The terms' columns add up (small terms first).
+#pragma unroll
+    for (int t = 0; t < G::NA; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = col < cols ? acc[t][i] : 0.f;
+        acc[t][i] = allreduce_sum<1, (CPH >= 4 ? 4 : 2)>(x) * (1.f / kPScale);
+      }
   }
+
+  // Wave totals per head to LDS (over the wave's digits), then the log-sum-exp
+  // merge of the waves.
+  const float l_tot =
+      allreduce_sum<16, 64>(allreduce_sum<1, (CPH >= 4 ? 4 : 2)>(l_run)) * (1.f / kPScale);
+  float* acc_w = reinterpret_cast<float*>(wave_s[w]) + hh * D;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (col == 0) {
 #pragma unroll
-  for (int h = 0; h < HG; ++h) {
+    for (int u = 0; u < G::NP; ++u)
 #pragma unroll
-    for (int k = 0; k < G::VCL; ++k) acc[h][k] = allreduce_sum<G::VPR, 64>(acc[h][k]);
-    if (lane < G::VPR) {
+      for (int i = 0; i < 4; ++i) {
+        float* dst = acc_w + u * 16 * G::CPP + (4 * grp + i) * G::CPP;
 #pragma unroll
-      for (int k = 0; k < G::VCL; ++k) acc_s[w][h][lane * G::VCL + k] = acc[h][k];
+        for (int j = 0; j < G::CPP; j += 4)
+          *reinterpret_cast<float4*>(dst + j) =
+              make_float4(acc[u * G::CPP + j][i], acc[u * G::CPP + j + 1][i],
+                          acc[u * G::CPP + j + 2][i], acc[u * G::CPP + j + 3][i]);
+      }
+    if (grp == 0) {
+      m_s[w][hh] = m_run;
+      l_s[w][hh] = l_tot;
     }
   }
   __syncthreads();
 
-  for (int idx = tid; idx < HG * D; idx += NT) {
+  // Four channels a thread: the waves' weights once, 16-byte reads and stores.
+  for (int idx = tid * 4; idx < HG * D; idx += NT * 4) {
     const int h = idx / D, d = idx % D;
     double ms = -INFINITY;
 #pragma unroll
     for (int i = 0; i < WAVES; ++i) ms = fmax(ms, m_s[i][h]);
-    float o = 0.f, l = 0.f;
+    float o[4] = {0.f, 0.f, 0.f, 0.f}, l = 0.f;
 #pragma unroll
     for (int i = 0; i < WAVES; ++i) {
-      const float e = (m_s[i][h] == -INFINITY) ? 0.f : exp2_of(m_s[i][h] - ms);
+      const float e =
+          (m_s[i][h] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((float)(m_s[i][h] - ms));
       l = __builtin_fmaf(e, l_s[i][h], l);
-      o = __builtin_fmaf(e, acc_s[i][h][d], o);
+      const float4 x = *reinterpret_cast<const float4*>(
+          reinterpret_cast<const float*>(wave_s[i]) + idx);
+      o[0] = __builtin_fmaf(e, x.x, o[0]);
+      o[1] = __builtin_fmaf(e, x.y, o[1]);
+      o[2] = __builtin_fmaf(e, x.z, o[2]);
+      o[3] = __builtin_fmaf(e, x.w, o[3]);
     }
     const int hq = h0 + h;
-    const int64_t pi = ((int64_t)b * a.num_q_heads + hq) * a.num_splits + split;
     if (a.final_out) {
-      store_elem(a.out, (int64_t)b * a.o_b + (int64_t)hq * a.o_h + d, a.out_dtype,
-                 o / fmaxf(l, 1e-10f));
+      const float r = fmaxf(l, 1e-10f);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        store_elem(a.out, (int64_t)b * a.o_b + (int64_t)hq * a.o_h + d + k, a.out_dtype, o[k] / r);
     } else {
-      a.ws_acc[pi * D + d] = o;
+      const int64_t pi = ((int64_t)b * a.num_q_heads + hq) * a.num_splits + split;
+      *reinterpret_cast<float4*>(a.ws_acc + pi * D + d) = make_float4(o[0], o[1], o[2], o[3]);
       if (d == 0) {
-        a.ws_ml[2 * pi] = ms;
+        a.ws_ml[2 * pi] = ms * 0.6931471805599453;   // natural log units
         a.ws_ml[2 * pi + 1] = (double)l;
       }
     }
@@ -400,14 +755,17 @@ hipError_t launch_decode_mfma(const DecodeArgs& a, int D, int v_dtype, int batch
     hipLaunchKernelGGL((decode_mfma_kernel<DD, VV, WW, HH>), grid, dim3(WW * 64), 0, st, a); \
     return hipGetLastError();                                                              \
   }
-#define FDI4_MF_H(WW, HH)                                                                 \
-  FDI4_MF(64, kVF32, WW, HH) FDI4_MF(128, kVF32, WW, HH)                                  \
-  FDI4_MF(64, kVF16, WW, HH) FDI4_MF(128, kVF16, WW, HH)                                  \
-  FDI4_MF(64, kVBF16, WW, HH) FDI4_MF(128, kVBF16, WW, HH)
+#define FDI4_MF_V(DD, WW, HH) \
+  FDI4_MF(DD, kVF32, WW, HH) FDI4_MF(DD, kVF16, WW, HH) FDI4_MF(DD, kVBF16, WW, HH)
+#define FDI4_MF_H(WW, HH) FDI4_MF_V(64, WW, HH) FDI4_MF_V(128, WW, HH)
   FDI4_MF_H(4, 2) FDI4_MF_H(8, 2) FDI4_MF_H(4, 4) FDI4_MF_H(8, 4)
-  // Eight heads per workgroup.
   FDI4_MF_H(4, 8) FDI4_MF_H(8, 8)
+  FDI4_MF_V(256, 4, 2) FDI4_MF_V(256, 4, 4)
+  // Eight waves of float32 values at D = 256 would spill registers.
+  FDI4_MF(256, kVF16, 8, 2) FDI4_MF(256, kVF16, 8, 4)
+  FDI4_MF(256, kVBF16, 8, 2) FDI4_MF(256, kVBF16, 8, 4)
 #undef FDI4_MF_H
+#undef FDI4_MF_V
 #undef FDI4_MF
   return hipErrorInvalidValue;
 }

@@ -64,6 +64,25 @@ struct StepAppend {
   int32_t* lens;                        // [B] the lengths, advanced by the last arriver
 };
 
+// Division of 0 <= n < 2^31 by a positive divisor fixed on the host:
+// n / d = (n * mul) >> shift with mul = ceil(2^shift / d), shift = 31 +
+// ceil(log2 d) (mul < 2^32; the excess mul * d - 2^shift < d <= 2^(shift - 31)
+// is too small to move the quotient). A 32-bit division on the device is some
+// 25 dependent instructions.
+struct FastDiv {
+  uint32_t mul;
+  int shift;
+};
+
+inline FastDiv make_fast_div(int d) {
+  int lg = 0;
+  while (((int64_t)1 << lg) < d) ++lg;
+  FastDiv f;
+  f.shift = 31 + lg;
+  f.mul = (uint32_t)((((uint64_t)1 << f.shift) + (uint64_t)d - 1) / (uint64_t)d);
+  return f;
+}
+
 // Split-K paged decode.
 struct DecodeArgs {
   const void* q;
@@ -82,6 +101,8 @@ struct DecodeArgs {
   const int32_t* page_lens;             // null: rows from seq_lens
   int64_t pl_b;
   int page_rows, pages_per_group, max_pages, hq_per_kv, num_pages;
+  FastDiv div_rows, div_cpp, div_ppg, div_hpk;  // by page_rows, 16-row chunks a page,
+                                        // pages_per_group, hq_per_kv
   int chunks_per_split, num_splits, num_q_heads;
   int final_out;                        // 1: normalized output; 0: split partials
   int waves;                            // wave64s per workgroup (4 or 8)
