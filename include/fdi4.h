@@ -157,6 +157,24 @@ int fdi4_quantize_paged(const float* k, int batch, int max_tokens, int64_t k_bat
                         int64_t k_head_stride, int64_t k_row_stride, int group_rows,
                         const fdi4_paged_cache* cache, hipStream_t stream);
 
+/* Start of sequences 0..batch-1 from dense keys k[b, h, t, :] (float32) and
+ * values v[b, h, t, :] (v_in_dtype, converted to the cache's value type as a cast
+ * rounds, to nearest even), element strides, channel stride 1, rows starting on
+ * 16-byte boundaries, for t < new_lens[b]: the keys as fdi4_quantize_paged writes
+ * them, the values to their pages, the float32 keys of each sequence's partial
+ * last group to k_stage[b, h, 0.., :] (as fdi4_append_paged expects them), new_lens
+ * to cache->seq_lens and the used entries of the rows of new_table to
+ * cache->page_table, in one launch. new_lens (int32 [batch]) and new_table (int32
+ * [batch, new_cols]) lie on the device, apart from the cache's arrays; lengths are
+ * clamped to [0, max_len] and max_len <= new_cols * page_rows. */
+int fdi4_prefill_paged(const float* k, int64_t k_batch_stride, int64_t k_head_stride,
+                       int64_t k_row_stride, const void* v, int v_in_dtype,
+                       int64_t v_batch_stride, int64_t v_head_stride, int64_t v_row_stride,
+                       int batch, int max_len, int group_rows, const int32_t* new_lens,
+                       const int32_t* new_table, int new_cols, float* k_stage,
+                       int64_t st_batch_stride, int64_t st_head_stride, int64_t st_row_stride,
+                       const fdi4_paged_cache* cache, hipStream_t stream);
+
 /* Decode-time append of one token per sequence b < batch at position
  * t = cache->seq_lens[b] (t < max_pages * page_rows; the caller has mapped
  * the page holding t in cache->page_table and advances seq_lens afterwards):

@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <vector>
 
@@ -295,6 +296,75 @@ void quantize_paged(torch::Tensor k, torch::Tensor seq_lens, torch::Tensor page_
   check_rc(fdi4_quantize_paged(k.data_ptr<float>(), (int)k.size(0), (int)k.size(2), k.stride(0),
                                k.stride(1), k.stride(2), (int)group_rows, &c, stream()),
            "quantize_paged");
+}
+
+// Sequences 0..B-1 of a cache started from k and v [B, kv_heads, T, D] (see
+// fdi4_prefill_paged). new_lens int32 [B] and new_table int32 [B, cols] are host
+// tensors; they go to the device in one copy from pinned memory, which waits for
+// nothing.
+void prefill_paged(torch::Tensor k, torch::Tensor v, torch::Tensor new_lens,
+                   torch::Tensor new_table, torch::Tensor k_stage, torch::Tensor k_pages,
+                   torch::Tensor v_pages, torch::Tensor k_scale, torch::Tensor k_zp,
+                   torch::Tensor page_table, torch::Tensor seq_lens, int64_t group_rows) {
+  CHECK_DEV(k);
+  CHECK_DEV(v);
+  CHECK_DEV(k_stage);
+  TORCH_CHECK(k.scalar_type() == torch::kFloat32 && k.dim() == 4 && k.stride(3) == 1,
+              "k must be float32 [batch, kv_heads, tokens, head_dim] with contiguous rows");
+  TORCH_CHECK(v.sizes() == k.sizes() && v.stride(3) == 1,
+              "v must have the shape of k, with contiguous rows");
+  TORCH_CHECK(k.size(1) == k_pages.size(1) && k.size(3) == k_pages.size(3) * 2 &&
+                  k_stage.dim() == 4 && k_stage.size(1) == k.size(1) &&
+                  k_stage.size(3) == k.size(3),
+              "k, k_stage and the cache must have the same kv_heads and head_dim");
+  TORCH_CHECK(k_stage.scalar_type() == torch::kFloat32 && k_stage.stride(3) == 1 &&
+                  k_stage.size(2) >= group_rows,
+              "k_stage must be float32 [batch, kv_heads, >= group_rows, head_dim]");
+  const int64_t B = k.size(0);
+  TORCH_CHECK(!new_lens.is_cuda() && !new_table.is_cuda() && new_lens.is_contiguous() &&
+                  new_table.is_contiguous() && new_lens.scalar_type() == torch::kInt32 &&
+                  new_table.scalar_type() == torch::kInt32 && new_lens.dim() == 1 &&
+                  new_table.dim() == 2 && new_lens.size(0) == B && new_table.size(0) == B,
+              "new_lens and new_table must be contiguous int32 host tensors with a row per "
+              "sequence");
+  TORCH_CHECK(k_stage.size(0) >= B && seq_lens.size(0) >= B && page_table.size(0) >= B &&
+                  k_scale.dim() == 4 && k_scale.size(0) >= B,
+              "k_stage, seq_lens, page_table and k_scale need a row per sequence");
+  TORCH_CHECK(group_rows > 0 && group_rows % k_pages.size(2) == 0,
+              "group_rows must be a multiple of page_rows");
+  const int64_t cols = new_table.size(1);
+  if (B == 0) return;
+  const int32_t* lens = new_lens.data_ptr<int32_t>();
+  int64_t max_len = 0;
+  for (int64_t b = 0; b < B; ++b) {
+    TORCH_CHECK(lens[b] >= 0 && lens[b] <= k.size(2), "lengths must lie in [0, tokens]");
+    max_len = std::max<int64_t>(max_len, lens[b]);
+  }
+  TORCH_CHECK(cols * k_pages.size(2) >= max_len && cols <= page_table.size(1),
+              "new_table must hold the pages of the longest sequence");
+  TORCH_CHECK(k_scale.size(2) * group_rows >= max_len, "k_scale has too few groups");
+  CHECK_SAME_DEVICE(k, v);
+  CHECK_SAME_DEVICE(k, k_stage);
+  CHECK_SAME_DEVICE(k, k_pages);
+  fdi4_paged_cache c = make_cache(k_pages, &v_pages, k_scale, k_zp, page_table, seq_lens,
+                                  c10::nullopt, group_rows / k_pages.size(2),
+                                  page_table.size(1));
+  const int vcode = dtype_code(v);
+  const DeviceGuard guard(k.device());
+  const int64_t n = B + B * cols;
+  auto host = torch::empty({n}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true));
+  int32_t* dst = host.data_ptr<int32_t>();
+  std::copy_n(lens, B, dst);
+  std::copy_n(new_table.data_ptr<int32_t>(), B * cols, dst + B);
+  auto meta = torch::empty({n}, seq_lens.options());
+  meta.copy_(host, /*non_blocking=*/true);
+  const int32_t* m = meta.data_ptr<int32_t>();
+  check_rc(fdi4_prefill_paged(k.data_ptr<float>(), k.stride(0), k.stride(1), k.stride(2),
+                              v.data_ptr(), vcode, v.stride(0), v.stride(1), v.stride(2), (int)B,
+                              (int)max_len, (int)group_rows, m, m + B, (int)cols,
+                              k_stage.data_ptr<float>(), k_stage.stride(0), k_stage.stride(1),
+                              k_stage.stride(2), &c, stream()),
+           "prefill_paged");
 }
 
 // One token per sequence appended at seq_lens[b] (see fdi4_append_paged);
@@ -688,6 +758,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "Fused online softmax + INT4 dequant attention over a shared page stream (HIP)");
   m.def("quantize_rows_into", &quantize_rows_into, "One-group INT4 quantization into views (HIP)");
   m.def("quantize_paged", &quantize_paged, "Grouped INT4 key quantization into packed pages (HIP)");
+  m.def("prefill_paged", &prefill_paged,
+        "Prompts into the cache: keys quantized, values paged, open groups staged (HIP)");
   m.def("append_paged", &append_paged,
         "Decode-time append: one token per sequence, open group re-quantized (HIP)");
   m.def("decode_paged", &decode_paged, "Split-K INT4 flash decoding over paged keys (HIP)");

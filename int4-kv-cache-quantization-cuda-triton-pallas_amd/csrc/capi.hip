@@ -338,6 +338,7 @@ QuantPagedArgs quant_args(const fdi4_paged_cache* cache) {
   a.s_h = cache->s_head_stride;
   a.s_g = cache->s_group_stride;
   a.page_rows = cache->page_rows;
+  a.div_rows = fdi4::make_fast_div(cache->page_rows);
   a.num_pages = cache->num_pages;
   a.max_tokens = 0;
   return a;
@@ -436,6 +437,59 @@ int append_paged_any(const float* k_new, int64_t kn_batch_stride, int64_t kn_hea
 }  // namespace
 
 extern "C" {
+
+int fdi4_prefill_paged(const float* k, int64_t k_batch_stride, int64_t k_head_stride,
+                  int64_t k_row_stride, const void* v, int v_in_dtype, int64_t v_batch_stride,
+                  int64_t v_head_stride, int64_t v_row_stride, int batch, int max_len,
+                  int group_rows, const int32_t* new_lens, const int32_t* new_table,
+                  int new_cols, float* k_stage, int64_t st_batch_stride, int64_t st_head_stride,
+                  int64_t st_row_stride, const fdi4_paged_cache* cache, hipStream_t stream) {
+  int rc = check_grouped_cache(cache, group_rows, true);
+  if (rc != hipSuccess) return rc;
+  if ((max_len > 0 && (!k || !v)) || !new_lens || !new_table || !k_stage || batch < 0 ||
+      batch > 65535 || max_len < 0 || new_cols < 0 || new_cols > cache->max_pages ||
+      (int64_t)new_cols * cache->page_rows < max_len)
+    return hipErrorInvalidValue;
+  if (v_in_dtype != FDI4_V_F32 && v_in_dtype != FDI4_V_F16 && v_in_dtype != FDI4_V_BF16)
+    return hipErrorInvalidValue;
+  const int D = cache->head_dim;
+  const int ieb = v_in_dtype == FDI4_V_F32 ? 4 : 2, veb = cache->v_dtype == FDI4_V_F32 ? 4 : 2;
+  // 16-byte loads of key and value rows, 16-byte stores of staging rows.
+  if (!aligned(k, 16) || k_batch_stride % 4 || k_head_stride % 4 || k_row_stride % 4 ||
+      !aligned(v, 16) || (v_batch_stride * ieb) % 16 || (v_head_stride * ieb) % 16 ||
+      (v_row_stride * ieb) % 16 || !aligned(k_stage, 16) || st_batch_stride % 4 ||
+      st_head_stride % 4 || st_row_stride % 4 || st_row_stride < D)
+    return hipErrorInvalidValue;
+  fdi4::PrefillArgs a;
+  a.q = quant_args(cache);
+  a.q.seq_lens = new_lens;
+  a.q.page_table = new_table;
+  a.q.pt_b = new_cols;
+  a.q.k = k;
+  a.q.k_b = k_batch_stride;
+  a.q.k_h = k_head_stride;
+  a.q.k_t = k_row_stride;
+  a.q.max_tokens = max_len;
+  a.v = static_cast<const uint8_t*>(v);
+  a.v_b = v_batch_stride * ieb;
+  a.v_h = v_head_stride * ieb;
+  a.v_t = v_row_stride * ieb;
+  a.v_in = v_in_dtype;
+  a.v_out = cache->v_dtype;
+  a.v_pages = static_cast<uint8_t*>(cache->v_pages);
+  a.vp_page = cache->v_page_stride * veb;
+  a.vp_head = cache->v_head_stride * veb;
+  a.vp_row = cache->v_row_stride * veb;
+  a.stage = k_stage;
+  a.st_b = st_batch_stride;
+  a.st_h = st_head_stride;
+  a.st_r = st_row_stride;
+  a.table_out = const_cast<int32_t*>(cache->page_table);
+  a.table_b = cache->pt_batch_stride;
+  a.lens_out = const_cast<int32_t*>(cache->seq_lens);
+  return fdi4::launch_prefill_paged(a, D, group_rows, batch, cache->num_kv_heads, max_len,
+                                    stream);
+}
 
 int fdi4_append_paged(const float* k_new, int64_t kn_batch_stride, int64_t kn_head_stride,
                       const void* v_new, int64_t vn_batch_stride, int64_t vn_head_stride,

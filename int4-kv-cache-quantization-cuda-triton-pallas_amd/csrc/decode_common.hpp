@@ -37,14 +37,6 @@ __device__ __forceinline__ float load_elem(const void* p, int64_t i, int dt) {
   return __uint_as_float((unsigned)u << 16);
 }
 
-// float32 -> bfloat16 bits, round to nearest even; NaN becomes the canonical
-// quiet NaN 0x7FC0 (as torch's conversion gives).
-__device__ __forceinline__ unsigned short bf16_rne(float x) {
-  const unsigned u = __float_as_uint(x);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (unsigned short)0x7FC0u;
-  return (unsigned short)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
-
 // Store x into element i of an output tensor of type dt, rounded to nearest
 // even for the 16-bit types.
 __device__ __forceinline__ void store_elem(void* p, int64_t i, int dt, float x) {
@@ -86,11 +78,6 @@ __device__ __forceinline__ void widen_values(const U32x4& v, float* f) {
 // load followed by a full vmcnt drain.
 __device__ __forceinline__ int ld_ro(const int32_t* p, int64_t i) {
   return ((const __attribute__((address_space(4))) int32_t*)p)[i];
-}
-
-// n / d for the divisor behind f (0 <= n < 2^31).
-__device__ __forceinline__ int fdiv(int n, FastDiv f) {
-  return (int)(((uint64_t)(uint32_t)n * f.mul) >> f.shift);
 }
 
 struct ChunkMeta {

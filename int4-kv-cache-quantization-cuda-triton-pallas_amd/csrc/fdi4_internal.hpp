@@ -13,6 +13,30 @@ enum VDtype : int { kVF32 = 0, kVF16 = 1, kVBF16 = 2 };
 // Element types of queries and outputs (the codes of fdi4_key_dtype).
 enum EDtype : int { kEF32 = 0, kEF16 = 1, kEBF16 = 2 };
 
+// Division of 0 <= n < 2^31 by a positive divisor fixed on the host:
+// n / d = (n * mul) >> shift with mul = ceil(2^shift / d), shift = 31 +
+// ceil(log2 d) (mul < 2^32; the excess mul * d - 2^shift < d <= 2^(shift - 31)
+// is too small to move the quotient). A 32-bit division on the device is some
+// 25 dependent instructions.
+struct FastDiv {
+  uint32_t mul;
+  int shift;
+};
+
+inline FastDiv make_fast_div(int d) {
+  int lg = 0;
+  while (((int64_t)1 << lg) < d) ++lg;
+  FastDiv f;
+  f.shift = 31 + lg;
+  f.mul = (uint32_t)((((uint64_t)1 << f.shift) + (uint64_t)d - 1) / (uint64_t)d);
+  return f;
+}
+
+// n / d for the divisor behind f (0 <= n < 2^31).
+__device__ __forceinline__ int fdiv(int n, FastDiv f) {
+  return (int)(((uint64_t)(uint32_t)n * f.mul) >> f.shift);
+}
+
 // Grouped paged quantizer: keys [B, H, T, D] (any strides, channel stride 1)
 // into packed pages and group scales.
 struct QuantPagedArgs {
@@ -27,8 +51,27 @@ struct QuantPagedArgs {
   float* zp;
   int64_t s_b, s_h, s_g;                // elements
   int page_rows;
+  FastDiv div_rows;                     // by page_rows
   int num_pages;                        // physical pages; table entries are clamped
   int max_tokens;                       // rows of k; sequence lengths are clamped to it
+};
+
+// Start of sequences from dense keys and values: the grouped quantizer (q, whose
+// page table and lengths are the new ones, read-only copies), the values into
+// their pages, the open groups' keys into the staging rows, and the new lengths
+// and page-table rows into the cache's.
+struct PrefillArgs {
+  QuantPagedArgs q;
+  const uint8_t* v;
+  int64_t v_b, v_h, v_t;                // bytes
+  int v_in, v_out;                      // VDtype of v and of the value pages
+  uint8_t* v_pages;
+  int64_t vp_page, vp_head, vp_row;     // bytes
+  float* stage;
+  int64_t st_b, st_h, st_r;             // elements
+  int32_t* table_out;
+  int64_t table_b;                      // elements
+  int32_t* lens_out;
 };
 
 // Decode-time append of one token per sequence (grouped quantizer re-run over
@@ -63,25 +106,6 @@ struct StepAppend {
   int32_t* arrive;                      // [B] arrival counters, zero between steps
   int32_t* lens;                        // [B] the lengths, advanced by the last arriver
 };
-
-// Division of 0 <= n < 2^31 by a positive divisor fixed on the host:
-// n / d = (n * mul) >> shift with mul = ceil(2^shift / d), shift = 31 +
-// ceil(log2 d) (mul < 2^32; the excess mul * d - 2^shift < d <= 2^(shift - 31)
-// is too small to move the quotient). A 32-bit division on the device is some
-// 25 dependent instructions.
-struct FastDiv {
-  uint32_t mul;
-  int shift;
-};
-
-inline FastDiv make_fast_div(int d) {
-  int lg = 0;
-  while (((int64_t)1 << lg) < d) ++lg;
-  FastDiv f;
-  f.shift = 31 + lg;
-  f.mul = (uint32_t)((((uint64_t)1 << f.shift) + (uint64_t)d - 1) / (uint64_t)d);
-  return f;
-}
 
 // Split-K paged decode.
 struct DecodeArgs {
@@ -141,6 +165,9 @@ size_t rows_workspace_bytes(int64_t rows, int C);
 
 hipError_t launch_quantize_paged(const QuantPagedArgs& a, int D, int group, int batch, int heads,
                                  int max_tokens, hipStream_t st);
+
+hipError_t launch_prefill_paged(const PrefillArgs& a, int D, int group, int batch, int heads,
+                                int max_len, hipStream_t st);
 
 hipError_t launch_append_paged(const AppendArgs& a, int D, int group, int batch, int heads,
                                hipStream_t st);

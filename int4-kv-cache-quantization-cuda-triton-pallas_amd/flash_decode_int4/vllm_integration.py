@@ -391,34 +391,33 @@ class INT4PagedSequenceCache:
         lens = np.asarray(seq_lens.cpu() if hasattr(seq_lens, "cpu") else seq_lens, np.int64)
         lens = lens.reshape(-1)
         self._check_prefill(k, v, lens)
-        B, _, T, _ = k.shape
+        B = k.shape[0]
         self._sync_if_stepped()
         for b in range(B):
             self._release(b)
-        try:
-            self._grow_all((b, int(lens[b])) for b in range(B))
-        except Exception:
-            self.seq_lens[:B] = 0  # the released slots are empty on the device too
-            raise
-        lens_t = torch.as_tensor(lens, dtype=torch.int32).cuda()
-        self.seq_lens[:B] = lens_t
+        # _check_prefill has seen to it that the pages exist: they leave the free
+        # list in one slice (the order successive pops would give).
+        need = (lens + self.page_rows - 1) // self.page_rows
+        ends = np.cumsum(need).tolist()
+        total = ends[-1] if B else 0
+        at = len(self._free) - total
+        taken = self._free[at:][::-1]
+        del self._free[at:]
+        for b, (n, end) in enumerate(zip(need.tolist(), ends)):
+            self._pages[b] = taken[end - n:end]
+        self._mapped[:B] = need * self.page_rows
         self._lens[:B] = lens
-        ops.quantize_int4_paged(k, self.seq_lens[:B], self.page_table[:B], self.k_pages,
-                                self.k_scale[:B], self.k_zp[:B], self.group_rows)
-        # Values: token t of sequence b -> row t % page_rows of physical page
-        # page_table[b, t // page_rows], gathered and scattered on the device.
-        if T and lens.any():
-            dev = self.seq_lens.device
-            t = torch.arange(T, device=dev)
-            bi, ti = torch.nonzero(t[None, :] < lens_t[:, None], as_tuple=True)
-            pages = self.page_table[bi, ti // self.page_rows].long()
-            self.v_pages[pages, :, ti % self.page_rows, :] = v[bi, :, ti, :].to(self.v_pages.dtype)
-        # Open groups: the float keys of each sequence's partial last group.
-        for b in range(B):
-            r = int(lens[b]) % self.group_rows
-            if r:
-                g0 = int(lens[b]) - r
-                self.k_stage[b, :, :r] = k[b, :, g0:g0 + r]
+        # One launch: the sequences' page-table rows and lengths go along with
+        # it, and the kernel writes them to the device arrays.
+        table = np.zeros((B, int(need.max(initial=0))), np.int32)
+        table[np.arange(table.shape[1]) < need[:, None]] = taken
+        es = v.element_size()
+        if v.stride(3) != 1 or v.data_ptr() % 16 or any((v.stride(i) * es) % 16 for i in range(3)):
+            v = v.clone(memory_format=torch.contiguous_format)
+        load_binding().prefill_paged(k, v, torch.from_numpy(lens.astype(np.int32)),
+                                     torch.from_numpy(table), self.k_stage, self.k_pages,
+                                     self.v_pages, self.k_scale, self.k_zp, self.page_table,
+                                     self.seq_lens, self.group_rows)
 
     def append(self, k_new, v_new) -> None:
         """Append one token to each of sequences 0..B-1: k_new float32 and v_new

@@ -1,0 +1,129 @@
+"""INT4PagedSequenceCache.prefill: pages, scales, staging rows, page table and
+lengths against the grouped quantizer and plain indexing, bit for bit."""
+
+import os
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+for p in (ROOT, os.path.join(ROOT, "int4-kv-cache-quantization-cuda-triton-pallas_amd")):
+    if p not in sys.path:
+        sys.path.insert(0, p)
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(c, k, v, lens):
+    import torch
+    from flash_decode_int4 import ops
+    B, H, T, D = k.shape
+    R, G = c.page_rows, c.group_rows
+    assert c.seq_lens[:B].tolist() == list(lens) == c.lengths()[:B].tolist()
+    kp, s, z = (torch.zeros_like(x) for x in (c.k_pages, c.k_scale, c.k_zp))
+    sl = torch.tensor(list(lens), dtype=torch.int32, device="cuda")
+    if T:
+        ops.quantize_int4_paged(k, sl, c.page_table[:B], kp, s[:B], z[:B], G)
+    for b, n in enumerate(lens):
+        pages = c.page_table[b, :-(-n // R)].long()
+        assert pages.tolist() == c._pages[b]
+        got = c.k_pages[pages].permute(1, 0, 2, 3).reshape(H, -1, D // 2)[:, :n]
+        want = kp[pages].permute(1, 0, 2, 3).reshape(H, -1, D // 2)[:, :n]
+        assert torch.equal(got, want)
+        g = -(-n // G)
+        assert torch.equal(c.k_scale[b, :, :g], s[b, :, :g])
+        assert torch.equal(c.k_zp[b, :, :g], z[b, :, :g])
+        got = c.v_pages[pages].permute(1, 0, 2, 3).reshape(H, -1, D)[:, :n]
+        want = v[b, :, :n].to(c.v_pages.dtype)
+        if want.dtype == torch.float32:
+            assert torch.equal(got.view(torch.int32), want.contiguous().view(torch.int32))
+        else:
+            assert torch.equal(got.contiguous().view(torch.int16),
+                               want.contiguous().view(torch.int16))
+        assert torch.equal(c.k_stage[b, :, :n % G], k[b, :, n - n % G:n])
+
+
+@pytest.mark.parametrize("D,R,G", [(64, 16, 64), (64, 1, 128), (128, 16, 128), (128, 8, 256),
+                                   (256, 32, 64), (256, 16, 128), (256, 256, 256)])
+@pytest.mark.parametrize("v_in,v_out", [("float32", "float32"), ("float16", "float16"),
+                                        ("float32", "bfloat16"), ("float32", "float16"),
+                                        ("bfloat16", "float16"), ("float16", "float32"),
+                                        ("bfloat16", "bfloat16")])
+def test_prefill(D, R, G, v_in, v_out):
+    import torch
+    from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
+    g = torch.Generator("cuda").manual_seed(D + R)
+    H, T = 3, 2 * G + 37
+    lens = [T, 0, 1, G, G + R, 2 * G - 1]
+    c = INT4PagedSequenceCache(sum(-(-n // R) for n in lens) + T // R + 2, H, D, len(lens) + 1, T + 5, R, G,
+                               v_out)
+    k = torch.randn(len(lens), H, T, D, device="cuda", generator=g)
+    v = torch.randn(len(lens), H, T, D, device="cuda", generator=g)
+    v[0, 0, 0, :8] = torch.tensor([float("inf"), -float("inf"), 65519.0, 65520.0, 1e-8, -6e-8,
+                                   3.4e38, -0.0], device="cuda")
+    v = v.to(getattr(torch, v_in))
+    before = [x.clone() for x in (c.k_stage, c.page_table)]
+    c.prefill(k, v, lens)
+    _check(c, k, v, lens)
+    # What no sequence uses stays as it was.
+    for b, n in enumerate(lens + [0]):
+        assert torch.equal(c.k_stage[b, :, n % G:], before[0][b, :, n % G:])
+        assert torch.equal(c.page_table[b, -(-n // R):], before[1][b, -(-n // R):])
+    # The same slots again, fewer and shorter sequences, pages handed back.
+    c.prefill(k[:2], v[:2], [7, T])
+    _check(c, k[:2], v[:2], [7, T])
+
+
+@pytest.mark.parametrize("how", ["transposed", "odd_offset", "expanded", "host_lens"])
+def test_prefill_of_views(how):
+    """Values of any strides (as before: plain indexing took them) and keys of
+    any aligned strides."""
+    import torch
+    from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
+    B, H, T, D = 2, 2, 150, 64
+    lens = [150, 33]
+    c = INT4PagedSequenceCache(40, H, D, B, T, 16, 64, "float16")
+    g = torch.Generator("cuda").manual_seed(1)
+    k = torch.randn(B, T, H, D, device="cuda", generator=g).permute(0, 2, 1, 3)
+    v = torch.randn(B, H, T, D, device="cuda", generator=g).half()
+    if how == "transposed":
+        v = torch.randn(B, H, D, T, device="cuda", generator=g).half().transpose(2, 3)
+    elif how == "odd_offset":
+        v = torch.randn(B * H * T * D + 3, device="cuda", generator=g).half()[3:].view(B, H, T, D)
+    elif how == "expanded":
+        v = v[:, :1].expand(B, H, T, D)
+    c.prefill(k, v, torch.tensor(lens) if how == "host_lens" else lens)
+    _check(c, k, v, lens)
+
+
+def test_prefill_of_nothing():
+    import torch
+    from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
+    c = INT4PagedSequenceCache(8, 2, 64, 2, 64, 16, 64, "float32")
+    k = torch.randn(2, 2, 40, 64, device="cuda")
+    c.prefill(k, k.clone(), [40, 3])
+    c.prefill(k[:0], k[:0], [])
+    _check(c, k, k, [40, 3])
+    c.prefill(k, k.clone(), [0, 0])
+    _check(c, k, k, [0, 0])
+    c.prefill(k[:, :, :0], k[:, :, :0], [0, 0])
+    assert sorted(c._free) == list(range(8))
+
+
+def test_prefill_from_two_streams():
+    """Each call's lengths and table travel in a buffer of its own: caches
+    filled from two streams at once hold what each was given."""
+    import torch
+    from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
+    g = torch.Generator("cuda").manual_seed(5)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    k = torch.randn(2, 4, 600, 128, device="cuda", generator=g)
+    caches = [INT4PagedSequenceCache(90, 4, 128, 2, 600, 16, 128, "bfloat16") for _ in streams]
+    torch.cuda.synchronize()
+    for i in range(6):
+        for c, st, n in zip(caches, streams, (600 - i, 77 + 31 * i)):
+            with torch.cuda.stream(st):
+                c.prefill(k, k, [n, 600 - n // 2])
+    torch.cuda.synchronize()
+    for c, n in zip(caches, (595, 232)):
+        _check(c, k, k, [n, 600 - n // 2])
