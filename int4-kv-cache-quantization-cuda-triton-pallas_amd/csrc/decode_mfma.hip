@@ -31,9 +31,8 @@
 //      four rows a lane group to the output of 16 channels x 16 columns. A
 //      float32 probability is the exact sum of three 8-bit (bfloat16) or
 //      11-bit (float16, scaled by 2^15) terms, which sit in different columns
-//      of the head (HG = 8: in the two halves of a 16x16x32 product), so the
-//      products are exact, their sums are float32, and one instruction does all
-//      terms. Only the final output adds the columns up.
+//      of the head (HG = 8: two columns, so two products), so the products are
+//      exact, their sums are float32, and one instruction does all terms. Only the final output adds the columns up.
 //      A non-finite value times an empty term is NaN where the float32 product
 //      is infinite: a wave that ends with a NaN runs its range again with the
 //      float32 products below.
@@ -59,8 +58,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
 template <int D, int VDT, int HG>
 struct MfmaGeo {
@@ -78,6 +75,8 @@ struct MfmaGeo {
   static constexpr int SZI = D / 2;                // 16-byte items in a scale+zp block
   static constexpr int SZL = (SZI + 63) / 64;      // scale+zp loads per lane
   static constexpr int DIGITS = 6;
+  // Chunks loaded ahead of the one consumed.
+  static constexpr int DEPTH = 1;
   // LDS per wave: the staged scale/zero-point block and the digits of a group
   // while the wave streams, its partial output afterwards.
   static constexpr int kDigBytes = DIGITS * HG * D;
@@ -148,25 +147,64 @@ __device__ __forceinline__ ChunkPos chunk_next(ChunkPos p, int cpp, int ppg) {
 }
 
 struct PosMeta {
-  int64_t phys;
+  unsigned phys;
   int r0, nval, group;
 };
 
-__device__ __forceinline__ PosMeta pos_meta(const DecodeArgs& a, int b, int T,
+// One sequence's page metadata. An absent table (null) is read at element 0 of
+// some valid array and the value dropped, which spares the chunk loop a branch
+// and its mask arithmetic.
+struct PageMeta {
+  const int32_t* table;
+  const int32_t* lens;
+  int table_mul, lens_mul;    // 1, or 0: absent
+};
+
+__device__ __forceinline__ PageMeta page_meta(const DecodeArgs& a, int b) {
+  PageMeta p;
+  const int32_t* any = reinterpret_cast<const int32_t*>(a.k_scale);
+  p.table = a.page_table ? a.page_table + (int64_t)b * a.pt_b : any;
+  p.lens = a.page_lens ? a.page_lens + (int64_t)b * a.pl_b : any;
+  p.table_mul = a.page_table ? 1 : 0;
+  p.lens_mul = a.page_lens ? 1 : 0;
+  return p;
+}
+
+__device__ __forceinline__ PosMeta pos_meta(const DecodeArgs& a, const PageMeta& pm, int T,
                                             const ChunkPos& p) {
   PosMeta m;
-  int rows;
-  if (a.page_lens) {
-    rows = min(max(ld_ro(a.page_lens, (int64_t)b * a.pl_b + p.lp), 0), a.page_rows);
-  } else {
-    rows = min(a.page_rows, T - p.lp * a.page_rows);
-  }
+  const int pg = ld_ro(pm.table, p.lp * pm.table_mul);
+  const int pl = ld_ro(pm.lens, p.lp * pm.lens_mul);
+  const int left = T - p.lp * a.page_rows;
+  const int rows = min(pm.lens_mul ? max(pl, 0) : left, a.page_rows);
   m.r0 = p.j * 16;
   m.nval = min(16, rows - m.r0);
-  const int pg = a.page_table ? ld_ro(a.page_table, (int64_t)b * a.pt_b + p.lp) : p.lp;
-  m.phys = (int64_t)min(max(pg, 0), a.num_pages - 1);
+  m.phys = (unsigned)min(max(pm.table_mul ? pg : p.lp, 0), a.num_pages - 1);
   m.group = p.group;
   return m;
+}
+
+// v_max without the quieting moves that fmax puts before operands of unknown
+// origin (the instruction quiets them itself).
+__device__ __forceinline__ float max_raw(float x, float y) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
+__device__ __forceinline__ double max_raw(double x, double y) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
+// Maximum over the four 16-lane groups: a swap of a register with its copy
+// leaves both groups' values in the two results.
+__device__ __forceinline__ float groups_max(float x) {
+  auto r = __builtin_amdgcn_permlane16_swap(f2u(x), f2u(x), false, false);
+  x = max_raw(u2f(r[0]), u2f(r[1]));
+  auto s = __builtin_amdgcn_permlane32_swap(f2u(x), f2u(x), false, false);
+  return max_raw(u2f(s[0]), u2f(s[1]));
 }
 
 template <int D, int VDT, int WAVES, int HG>
@@ -210,6 +248,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   }
 
   const int cpp = (a.page_rows + 15) >> 4, ppg = a.pages_per_group;
+  const PageMeta pgm = page_meta(a, b);
   const int T = seq_len_of(a, b);
   const int n_chunks = pages_of(a, T) * cpp;
   const int c_begin = split * a.chunks_per_split;
@@ -237,8 +276,22 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   const uint8_t* kbase_h = a.k_pages + (int64_t)hk * a.k_head;
   const uint8_t* vbase_h = reinterpret_cast<const uint8_t*>(a.v_pages) +
                            (int64_t)hk * a.v_head * G::VEB;
-  const unsigned k_lane = grp * (D / 8), v_lane = n16 * G::PB;
   const unsigned krow_b = (unsigned)a.k_row, vrow_b = (unsigned)(a.v_row * G::VEB);
+  // Offsets of this lane's key row and value rows in a full chunk; a partial one
+  // takes the smaller of these and the last valid row's.
+  const unsigned k_lane = grp * (D / 8), v_lane = n16 * G::PB;
+  const unsigned k_full = k_lane + n16 * krow_b;
+  unsigned v_full[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v_full[i] = v_lane + (4 * grp + i) * vrow_b;
+  // Scale/zero-point block of a group: items 0..D/4-1 are scale[4e..4e+3], items
+  // D/4..D/2-1 are zp. Lanes past the block reload an in-range item.
+  const float* sz_src[G::SZL];
+#pragma unroll
+  for (int i = 0; i < G::SZL; ++i) {
+    const int e = (i * 64 + lane) % G::SZI;
+    sz_src[i] = e < D / 4 ? sbase + 4 * e : zbase + 4 * (e - D / 4);
+  }
 
   struct Buf {
     unsigned k[G::KW];
@@ -246,20 +299,19 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   };
 
   auto load_sz = [&](const PosMeta& m, U32x4* sz) __attribute__((always_inline)) {
-    const int64_t off = (int64_t)m.group * a.s_g + m.phys * a.s_p;
+    const int64_t off = (uint64_t)(unsigned)m.group * (uint64_t)a.s_g +
+                        (uint64_t)m.phys * (uint64_t)a.s_p;
 #pragma unroll
-    for (int i = 0; i < G::SZL; ++i) {
-      const int e = (i * 64 + lane) % G::SZI;
-      const float* src = (e < D / 4) ? (sbase + off + 4 * e) : (zbase + off + 4 * (e - D / 4));
-      sz[i] = ld16(src);
-    }
+    for (int i = 0; i < G::SZL; ++i) sz[i] = ld16(sz_src[i] + off);
   };
 
   // Rows past the valid count are loaded from the last valid row (never out of
   // bounds); their probabilities are 0.
   auto load_chunk = [&](const PosMeta& m, int nval, Buf& f) __attribute__((always_inline)) {
-    const uint8_t* kb = kbase_h + m.phys * a.k_page + (int64_t)m.r0 * a.k_row;
-    const unsigned ko = k_lane + (unsigned)max(min(n16, nval - 1), 0) * krow_b;
+    const unsigned last = (unsigned)max(nval - 1, 0);
+    const uint8_t* kb = kbase_h + ((uint64_t)m.phys * (uint64_t)a.k_page +
+                                   (uint64_t)(unsigned)m.r0 * krow_b);
+    const unsigned ko = min(k_full, k_lane + last * krow_b);
     constexpr int KL = G::KW < 4 ? G::KW : 4;
 #pragma unroll
     for (int i = 0; i < G::KW / KL; ++i) {
@@ -267,10 +319,12 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
 #pragma unroll
       for (int k = 0; k < KL; ++k) f.k[KL * i + k] = x.w[k];
     }
-    const uint8_t* vb = vbase_h + (m.phys * a.v_page + (int64_t)m.r0 * a.v_row) * G::VEB;
+    const uint8_t* vb = vbase_h + ((uint64_t)m.phys * (uint64_t)(a.v_page * G::VEB) +
+                                   (uint64_t)(unsigned)m.r0 * vrow_b);
+    const unsigned v_last = v_lane + last * vrow_b;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const unsigned vo = v_lane + (unsigned)max(min(4 * grp + i, nval - 1), 0) * vrow_b;
+      const unsigned vo = min(v_full[i], v_last);
 #pragma unroll
       for (int u = 0; u < G::NP; ++u) {
         const KVec<G::PB / 4> x = load_k<G::PB / 4>(vb + (vo + 16 * G::PB * u));
@@ -381,11 +435,17 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   // Column sums of a digit pair: lane pairs (even column: high digit) exchange
   // rows, the even lane keeping rows 0 and 2 of its four, the odd one 1 and 3.
   const int wsh = odd ? 0 : 8;
+  // Selects as bit selects under lane masks: a ternary over vector elements
+  // becomes an indexed access, five instructions for one.
+  const int m_odd = odd ? -1 : 0, m_hi2 = hi2 ? -1 : 0;
+  auto sel = [](int m, int x, int y) __attribute__((always_inline)) {
+    return (m & x) | (~m & y);
+  };
   auto pair_rows = [&](const v4i& d, int* r) __attribute__((always_inline)) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      const int keep = (odd ? d[2 * k + 1] : d[2 * k]) << wsh;
-      const int send = (odd ? d[2 * k] : d[2 * k + 1]) << wsh;
+      const int keep = sel(m_odd, d[2 * k + 1], d[2 * k]) << wsh;
+      const int send = sel(m_odd, d[2 * k], d[2 * k + 1]) << wsh;
       r[k] = keep + (int)dpp<0xB1>((unsigned)send);
     }
   };
@@ -419,14 +479,14 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     } else {
       int p[2];
       pair_rows(ds[0], p);
-      const int own = hi2 ? p[1] : p[0];
-      const int oth = (int)dpp<0x4E>((unsigned)(hi2 ? p[0] : p[1]));
+      const int own = sel(m_hi2, p[1], p[0]);
+      const int oth = (int)dpp<0x4E>((unsigned)sel(m_hi2, p[0], p[1]));
       double s;
       if constexpr (CPH == 4) {
         int r[2];
         pair_rows(ds[1], r);
         s = __builtin_fma((double)own, w_own,
-                          __builtin_fma((double)oth, w_oth, (double)(hi2 ? r[1] : r[0])));
+                          __builtin_fma((double)oth, w_oth, (double)sel(m_hi2, r[1], r[0])));
       } else {
         s = __builtin_fma((double)own, w_own, (double)oth * w_oth);
         s += xchg4_dpp(s);
@@ -478,7 +538,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   auto value_16 = [&](const Buf& f, const float* x) __attribute__((always_inline)) {
     unsigned bt[4];
     if constexpr (CPH == 2) {
-      // Column 0: first and second term; column 1: third term and nothing.
+      // Column 0: first, then second term; column 1: third, then nothing.
       float ta[4], tb[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -511,16 +571,10 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
         const unsigned a0 = __builtin_amdgcn_perm(f.v[1][u][j / 2], f.v[0][u][j / 2], sel);
         const unsigned a1 = __builtin_amdgcn_perm(f.v[3][u][j / 2], f.v[2][u][j / 2], sel);
         v4f& t = acc[u * G::CPP + j];
-        if constexpr (CPH == 2) {
-          const U32x4 av = {a0, a1, a0, a1}, bv = {bt[0], bt[1], bt[2], bt[3]};
-          if constexpr (VDT == kVF16)
-            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, av),
-                                                       __builtin_bit_cast(v8h, bv), t, 0, 0, 0);
-          else
-            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, av),
-                                                        __builtin_bit_cast(v8b, bv), t, 0, 0, 0);
-        } else {
-          const uint2 av = make_uint2(a0, a1), bv = make_uint2(bt[0], bt[1]);
+        const uint2 av = make_uint2(a0, a1);
+#pragma unroll
+        for (int q = 0; q < (CPH == 2 ? 2 : 1); ++q) {
+          const uint2 bv = make_uint2(bt[2 * q], bt[2 * q + 1]);
           if constexpr (VDT == kVF16)
             t = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, av),
                                                       __builtin_bit_cast(v4h, bv), t, 0, 0, 0);
@@ -536,14 +590,15 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   auto consume = [&](const Buf& f, int nval, bool wide) __attribute__((always_inline)) {
     double lg[RN];
     logits(f, lg);
-    float mloc = -INFINITY;
+    float mc = -INFINITY;
 #pragma unroll
     for (int k = 0; k < RN; ++k) {
       lg[k] = lrow + 2 * k < nval ? lg[k] : -INFINITY;
-      mloc = fmaxf(mloc, (float)lg[k]);
+      mc = max_raw(mc, (float)lg[k]);
     }
-    float mc = allreduce_max_f<1, (CPH >= 4 ? 4 : 2)>(mloc);
-    mc = allreduce_max_f<16, 64>(mc);
+    mc = max_raw(mc, xchg<1>(mc));
+    if constexpr (CPH >= 4) mc = max_raw(mc, xchg<2>(mc));
+    mc = groups_max(mc);
     // The shift: the float32 maximum of the rounded logits, raised by two of
     // its ulps so that no probability exceeds 1 -- or, where two ulps are more
     // than a quarter, the double maximum itself.
@@ -553,7 +608,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
       if constexpr (RN > 1) mx = fmax(mx, lg[RN - 1]);
       mx = allreduce_max<16, 64>(allreduce_max<1, (CPH >= 4 ? 4 : 2)>(mx));
     }
-    const double m_new = fmax(m_run, mx);
+    const double m_new = max_raw(m_run, mx);
     const float corr = __builtin_amdgcn_exp2f((float)(m_run - m_new));
     m_run = m_new;
     float p[RN], psum = 0.f;
@@ -588,44 +643,48 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     }
   };
 
-  // One step: (1) rebuild for a new scale group, (2) prefetch chunk c+1 (one row
-  // of the last chunk on the last step, so that every step issues the same loads
-  // and the wait counts stay exact), (3) read the page-table entry of chunk c+2
-  // on the scalar unit, (4) consume chunk c. Called alternately with the two
-  // buffers swapped, so no register copy waits on the prefetch.
+  // One step: (1) rebuild for a new scale group, (2) load the next chunk's scale
+  // block and the chunk DEPTH ahead (past the end one row of the last chunk, so
+  // that every step issues the same loads and the wait counts stay exact),
+  // (3) read the page-table entry of the chunk after that on the scalar unit,
+  // (4) consume chunk c. Called with the DEPTH + 1 buffers in turn, so no
+  // register copy waits on a load.
+  constexpr int DEPTH = G::DEPTH;
   int c = wc0;
   ChunkPos np{};
-  PosMeta cm{}, nm{};
+  PosMeta mq[DEPTH + 1];      // of chunks c .. c + DEPTH
   U32x4 sz[G::SZL];
-  auto advance = [&](int ci) __attribute__((always_inline)) {
+  auto next_meta = [&](int ci) __attribute__((always_inline)) -> PosMeta {
     if (ci < wc1) np = chunk_next(np, cpp, ppg);
+    return pos_meta(a, pgm, T, np);
   };
   auto step = [&](const Buf& f, Buf& nf) __attribute__((always_inline)) -> bool {
-    if (cm.group != cur_group) {
+    if (mq[0].group != cur_group) {
       rebuild(sz);
-      cur_group = cm.group;
+      cur_group = mq[0].group;
     }
-    const bool last = c + 1 >= wc1;
-    load_sz(nm, sz);
-    load_chunk(nm, last ? 1 : nm.nval, nf);
-    advance(c + 2);
-    const PosMeta nnm = pos_meta(a, b, T, np);
-    if (cm.nval > 0) consume(f, cm.nval, false);
+    load_sz(mq[1], sz);
+    load_chunk(mq[DEPTH], c + DEPTH >= wc1 ? 1 : mq[DEPTH].nval, nf);
+    const PosMeta ahead = next_meta(c + DEPTH + 1);
+    if (mq[0].nval > 0) consume(f, mq[0].nval, false);
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) mq[i] = mq[i + 1];
+    mq[DEPTH] = ahead;
     c += 1;
-    cm = nm;
-    nm = nnm;
-    return last;
+    return c >= wc1;
   };
 
   const bool has_work = wc0 < wc1;
-  Buf fa, fb;
+  Buf f[DEPTH + 1];
   auto first_loads = [&]() __attribute__((always_inline)) {
     np = chunk_pos(a, wc0, cpp);
-    cm = pos_meta(a, b, T, np);
-    advance(wc0 + 1);
-    nm = pos_meta(a, b, T, np);
-    load_sz(cm, sz);
-    load_chunk(cm, cm.nval, fa);
+    mq[0] = pos_meta(a, pgm, T, np);
+#pragma unroll
+    for (int i = 1; i <= DEPTH; ++i) mq[i] = next_meta(wc0 + i);
+    load_sz(mq[0], sz);
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i)
+      load_chunk(mq[i], wc0 + i >= wc1 ? 1 : mq[i].nval, f[i]);
   };
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -641,8 +700,14 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   __syncthreads();
   if (has_work) {
     while (true) {
-      if (step(fa, fb)) break;
-      if (step(fb, fa)) break;
+      if constexpr (DEPTH == 1) {
+        if (step(f[0], f[1])) break;
+        if (step(f[1], f[0])) break;
+      } else {
+        if (step(f[0], f[2])) break;
+        if (step(f[1], f[0])) break;
+        if (step(f[2], f[1])) break;
+      }
     }
   }
 
@@ -663,14 +728,14 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
       cols = 1;
       ChunkPos p = chunk_pos(a, wc0, cpp);
       for (int ci = wc0; ci < wc1; ++ci) {
-        const PosMeta m = pos_meta(a, b, T, p);
+        const PosMeta m = pos_meta(a, pgm, T, p);
         load_sz(m, sz);
-        load_chunk(m, m.nval, fa);
+        load_chunk(m, m.nval, f[0]);
         if (m.group != cur_group) {
           rebuild(sz);
           cur_group = m.group;
         }
-        if (m.nval > 0) consume(fa, m.nval, true);
+        if (m.nval > 0) consume(f[0], m.nval, true);
         p = chunk_next(p, cpp, ppg);
       }
     }
@@ -760,10 +825,7 @@ hipError_t launch_decode_mfma(const DecodeArgs& a, int D, int v_dtype, int batch
 #define FDI4_MF_H(WW, HH) FDI4_MF_V(64, WW, HH) FDI4_MF_V(128, WW, HH)
   FDI4_MF_H(4, 2) FDI4_MF_H(8, 2) FDI4_MF_H(4, 4) FDI4_MF_H(8, 4)
   FDI4_MF_H(4, 8) FDI4_MF_H(8, 8)
-  FDI4_MF_V(256, 4, 2) FDI4_MF_V(256, 4, 4)
-  // Eight waves of float32 values at D = 256 would spill registers.
-  FDI4_MF(256, kVF16, 8, 2) FDI4_MF(256, kVF16, 8, 4)
-  FDI4_MF(256, kVBF16, 8, 2) FDI4_MF(256, kVBF16, 8, 4)
+  FDI4_MF_V(256, 4, 2) FDI4_MF_V(256, 4, 4)   // four waves only, see plan_decode
 #undef FDI4_MF_H
 #undef FDI4_MF_V
 #undef FDI4_MF
