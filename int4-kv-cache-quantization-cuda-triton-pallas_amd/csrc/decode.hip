@@ -106,18 +106,6 @@ __device__ __forceinline__ void step_arrive(const DecodeArgs& a, int b, int lane
   }
 }
 
-// One split's term of the log-sum-exp merge of an output element: split
-// maximum m (-inf: the split holds no rows and adds nothing), its sum of
-// probabilities lraw and weighted value acc, against the maximum ms over the
-// splits.
-__device__ __forceinline__ void merge_term(double m, double ms, float acc, double lraw, float& o,
-                                           float& l) {
-  if (m == -INFINITY) return;
-  const float e = exp2_of(m - ms);
-  o = __builtin_fmaf(e, acc, o);
-  l = __builtin_fmaf(e, (float)lraw, l);
-}
-
 // Waves of a decode workgroup that only re-quantize: the fused serving step
 // adds four, which re-quantize the open group while the decode waves stream,
 // with four decode waves, and with eight where three waves per SIMD fit in
@@ -525,48 +513,76 @@ decode_kernel(DecodeArgs a) {
   }
 }
 
-// Log-sum-exp merge of the split partials: grid (Hq, B), one thread per
-// channel. Split s adds nothing when its maximum is -inf (no rows); the
-// others add exp(m_s - max) times their values and sums, in split order. Up
-// to eight splits every partial a thread needs is loaded in one round
-// (indices clamped to the last split, the extra loads unused); more splits
-// take the loop.
+// Log-sum-exp merge of the split partials: grid (Hq, B), one wave, D / 64
+// channels a lane. Split s adds nothing when its maximum is -inf (no rows); the
+// others add exp(m_s - max) times their values and sums. The partials of eight
+// splits are in flight at a time; lane j holds split j's maximum and sum and
+// computes its weight once, and the lanes take the weights as scalars.
+//
+// Bound by latency (the launch, its arguments, one round to partials that other
+// XCDs wrote, and the instruction fetch of code that runs once), so the code is
+// short: against a thread per channel, each computing every weight, D = 256 B4
+// Hq16 with eight splits 6.5 -> 4.0 us (the call 19.4 -> 16.0), D = 128 B8 Hq32
+// with four 4.6 -> 4.4. (Merging in the decode kernel by the last workgroup to
+// arrive was no faster than this launch: 32.0 us against 32.3 at B8 Hkv8 Hq32
+// T8192, 14.1 against 13.6 for the shared stream of 2048 rows.)
 template <int D>
-__global__ __launch_bounds__(D) void merge_kernel(const float* __restrict__ ws_acc,
-                                                  const double* __restrict__ ws_ml, int hq,
-                                                  int splits, void* __restrict__ out,
-                                                  int out_dtype, int64_t o_b, int64_t o_h) {
-  const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
+__global__ __launch_bounds__(64) void merge_kernel(const float* __restrict__ ws_acc,
+                                                   const double* __restrict__ ws_ml, int hq,
+                                                   int splits, void* __restrict__ out,
+                                                   int out_dtype, int64_t o_b, int64_t o_h) {
+  constexpr int CH = D / 64, NB = 8;
+  struct alignas(4 * CH) Ch {
+    float v[CH];
+  };
+  const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
   const int64_t p0 = ((int64_t)b * hq + h) * splits;
+  const Ch* acc = reinterpret_cast<const Ch*>(ws_acc + p0 * D) + lane;
+  const double2* ml = reinterpret_cast<const double2*>(ws_ml + 2 * p0);
   double ms = -INFINITY;
-  float o = 0.f, l = 0.f;
-  if (splits <= 8) {
-    double mv[8], lv[8];
-    float av[8];
+  float l = 0.f;
+  Ch o = {};
+#pragma unroll 1
+  for (int s0 = 0; s0 < splits; s0 += NB) {
+    const int mine = s0 + (lane & (NB - 1));
+    double2 x = ml[min(mine, splits - 1)];
+    Ch av[NB];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int64_t p = p0 + min(j, splits - 1);
-      mv[j] = ws_ml[2 * p];
-      lv[j] = ws_ml[2 * p + 1];
-      av[j] = ws_acc[p * D + d];
+    for (int j = 0; j < NB; ++j) av[j] = acc[(int64_t)min(s0 + j, splits - 1) * 64];
+    if (mine >= splits) x = make_double2(-INFINITY, 0.0);
+    // The running maximum (over eight lanes, the same in all), and what it does
+    // to the sums of earlier rounds.
+    double mr = fmax(x.x, xchg<1>(x.x));
+    mr = fmax(mr, xchg<2>(mr));
+    mr = fmax(fmax(mr, xchg<4>(mr)), ms);
+    const bool live = x.x != -INFINITY;
+    const float e = live ? exp2_of(x.x - mr) : 0.f;
+    if (s0 > 0 && ms != -INFINITY) {
+      const float c = exp2_of(ms - mr);
+      l *= c;
+#pragma unroll
+      for (int k = 0; k < CH; ++k) o.v[k] *= c;
     }
-    // Each value is used only under its split's condition; without this the
-    // compiler moves every load into its branch, one memory round per split.
+    ms = mr;
+    float lj = live ? e * (float)x.y : 0.f;
+    lj += xchg<1>(lj);
+    lj += xchg<2>(lj);
+    l += lj + xchg<4>(lj);
+    const unsigned mask = (unsigned)__builtin_amdgcn_ballot_w64(live) & 255u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) asm volatile("" ::"v"(av[j]));
+    for (int j = 0; j < NB; ++j) {
+      // An empty split's values are not read (they may be anything).
+      if (mask >> j & 1u) {
+        const float ej = u2f((unsigned)__builtin_amdgcn_readlane((int)f2u(e), j));
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < splits) ms = fmax(ms, mv[j]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < splits) merge_term(mv[j], ms, av[j], lv[j], o, l);
-  } else {
-    for (int s = 0; s < splits; ++s) ms = fmax(ms, ws_ml[2 * (p0 + s)]);
-    for (int s = 0; s < splits; ++s)
-      merge_term(ws_ml[2 * (p0 + s)], ms, ws_acc[(p0 + s) * D + d], ws_ml[2 * (p0 + s) + 1], o,
-                 l);
+        for (int k = 0; k < CH; ++k) o.v[k] = __builtin_fmaf(ej, av[j].v[k], o.v[k]);
+      }
+    }
   }
-  store_elem(out, (int64_t)b * o_b + (int64_t)h * o_h + d, out_dtype, o / fmaxf(l, 1e-10f));
+  const float r = fmaxf(l, 1e-10f);
+#pragma unroll
+  for (int k = 0; k < CH; ++k)
+    store_elem(out, (int64_t)b * o_b + (int64_t)h * o_h + lane * CH + k, out_dtype, o.v[k] / r);
 }
 
 hipError_t launch_decode(const DecodeArgs& a, int D, int v_dtype, int batch, hipStream_t st) {
@@ -596,7 +612,7 @@ hipError_t launch_merge(const float* ws_acc, const double* ws_ml, int batch, int
   dim3 grid(hq, batch);
 #define FDI4_MRG(DD)                                                                         \
   if (D == DD) {                                                                             \
-    hipLaunchKernelGGL((merge_kernel<DD>), grid, dim3(DD), 0, st, ws_acc, ws_ml, hq, splits, \
+    hipLaunchKernelGGL((merge_kernel<DD>), grid, dim3(64), 0, st, ws_acc, ws_ml, hq, splits, \
                        out, out_dtype, o_b, o_h);                                            \
     return hipGetLastError();                                                                \
   }
