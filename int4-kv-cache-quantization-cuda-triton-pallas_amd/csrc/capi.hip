@@ -22,14 +22,15 @@ namespace {
 using fdi4::DecodeArgs;
 using fdi4::QuantPagedArgs;
 
-// Decode launch shape. A workgroup has 4 or 8 wave64s; the split count is the
-// smallest that gives about kTargetWaves resident waves (8 per CU on 256 CUs,
-// the occupancy the decode kernel's ~200 VGPRs allow), so that with enough
-// (sequence, head) streams no split -- and no merge kernel -- is needed.
-// FDI4_TUNE_DECODE_WAVES and FDI4_TUNE_DECODE_TARGET_WAVES override the choice.
+// Decode launch shape. A workgroup has 4 or 8 wave64s, eight as soon as each
+// gets kMinChunksPerWave 16-row chunks; the split count comes from an estimate of
+// the call's time (pick_splits). FDI4_TUNE_DECODE_WAVES overrides the waves;
+// FDI4_TUNE_DECODE_TARGET_WAVES replaces the estimate by the smallest count that
+// gives so many waves.
 constexpr int kTargetWaves = 2048;
 constexpr int kMinChunksPerWave = 4;
-constexpr int kMaxGroupedSplits = 8;
+constexpr int kMaxSplits = 64;
+constexpr int64_t kCUs = 256;
 constexpr size_t kAlign = 256;
 
 inline size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
@@ -42,6 +43,10 @@ int padded_head_dim(int d) { return d <= 64 ? 64 : (d <= 128 ? 128 : 256); }
 
 int chunks_per_seq(const fdi4_paged_cache* c) {
   return c->max_pages * ceil_div(c->page_rows, 16);
+}
+
+int chunks_per_group(const fdi4_paged_cache* c) {
+  return c->pages_per_group * ceil_div(c->page_rows, 16);
 }
 
 // Launch-shape overrides set through fdi4_set_tuning (0 = automatic). Atomic
@@ -127,13 +132,72 @@ bool one_wave_per_simd(int d, int v_dtype, int64_t streams) {
   return d == 128 && v_dtype == FDI4_V_F32 && streams * 4 <= kTargetWaves;
 }
 
-// Launch shape of a decode: heads per workgroup, waves per workgroup (the
-// grouped kernel at D=256 has registers for four), and the split count that
-// gives about kTargetWaves waves over the (sequence, head group) streams. The
-// fused serving step takes the same shape (and so gives the same bits as the
-// append and the decode); with four decode waves its kernel adds four helper
-// waves that re-quantize the open group meanwhile.
-DecodePlan plan_decode(int batch, int hq, int hq_per_kv, int d, int v_dtype, int chunks) {
+// Split count of a decode: the one with the smallest estimated time, over
+// `streams` (sequence, head group) streams of `chunks` 16-row chunks.
+//
+//   rounds  workgroups fill the 256 CUs (two four-wave ones each at D <= 128) in
+//           whole rounds: 320 eight-wave workgroups take as long as 512, since 64
+//           CUs hold two. Splits that spill into another round were the largest
+//           loss of a fixed wave target. (The float32 per-head kernel counts one
+//           workgroup a CU: the serving step adds four waves to it, and took 35.0
+//           us at B2 H32 T2032 with two against 24.7.)
+//   chunk   a wave's time per chunk: its own (measured with few workgroups: 0.85
+//           us in the matrix-core kernel, 1.0 in the per-head one, 0.85 at D =
+//           64; 1.0 and 1.9 at D = 256), or its share of memory when many waves
+//           stream (7.5 bytes/ps from HBM, 11 where the whole cache is small
+//           enough to stay in the last-level cache between calls).
+//   fixed   6 us of launch, first loads and the waves' merge, 4 of them again for
+//           each further round; the split merge 2.6 us and 0.05 per split.
+//
+// Estimates within 2 % count as equal, and then the count with more workgroups is
+// taken. With one q-head per kv-head a count whose splits hold whole scale groups
+// is preferred by 0.5 us: the serving step appends in the same launch there.
+//
+// Measured against the smallest count that gives 2048 waves (us per call): B5 H32
+// T1500 float16 26.3 -> 18.9, B40 H4 T2500 float16 36.9 -> 29.7, B12 H16 D256 T1200
+// float32 54.2 -> 45.3, B3 H32 D256 T2000 float16 38.0 -> 27.9, B40 Hkv4 Hq32 T600
+// float32 24.0 -> 17.0, B6 Hkv8 Hq16 D256 T2500 float16 26.5 -> 19.6. Lengths are
+// not known here: where they are ragged, a count that overfills the CUs with
+// workgroups of short sequences can be better (B30 Hkv2 Hq8 float32 steps to 6000
+// rows 36.3 -> 37.8).
+int pick_splits(int64_t streams, int waves, int chunks, int d, int v_dtype, bool mfma,
+                bool grouped, bool one_head, int group_chunks) {
+  const double veb = v_dtype == FDI4_V_F32 ? 4.0 : 2.0;
+  const double chunk_bytes = 16.0 * d * (0.5 + veb);
+  const double alone = mfma ? (d == 256 ? 1.0 : 0.85) : (d == 256 ? 1.9 : d == 64 ? 0.85 : 1.0);
+  const double rate = (double)streams * chunks * chunk_bytes > 128e6 ? 7.5e6 : 11e6;   // bytes/us
+  const bool pairs = waves == 4 && d <= 128 && !(one_head && d == 128 && v_dtype == FDI4_V_F32);
+  const int64_t slots = pairs ? 2 * kCUs : kCUs;
+  // At least one chunk a wave in the grouped kernels, four in the per-head one.
+  const int per_wave = grouped ? 1 : kMinChunksPerWave;
+  const int most = std::max(1, std::min(chunks / (waves * per_wave), kMaxSplits));
+  int best = 1;
+  double best_t = 0.0;
+  for (int s = 1; s <= most; ++s) {
+    const int per_split = ceil_div(chunks, s);
+    if (s > 1 && ceil_div(chunks, per_split) != s) continue;   // leaves splits empty
+    const int64_t wgs = streams * s;
+    const int64_t rounds = (wgs + slots - 1) / slots;
+    // The fullest CUs set the pace.
+    const int64_t busy = wgs <= kCUs ? wgs : slots;
+    const double chunk = std::max(alone, (double)busy * waves * chunk_bytes / rate);
+    double t = 2.0 + rounds * (4.0 + chunk * per_split / waves);
+    if (s > 1) t += 2.6 + 0.05 * s;
+    if (s > 1 && one_head && per_split % group_chunks != 0) t += 0.5;
+    if (s == 1 || t < best_t * (wgs <= slots ? 1.02 : 1.0)) {
+      best = s;
+      best_t = s == 1 ? t : std::min(t, best_t);
+    }
+  }
+  return best;
+}
+
+// Launch shape of a decode: heads per workgroup, waves per workgroup and split
+// count. The fused serving step takes the same shape (and so gives the same
+// bits as the append and the decode); with four decode waves its kernel adds
+// four helper waves that re-quantize the open group meanwhile.
+DecodePlan plan_decode(int batch, int hq, int hq_per_kv, int d, int v_dtype, int chunks,
+                       int group_chunks) {
   DecodePlan p;
   p.mfma = use_mfma() ? 1 : 0;
   p.heads_per_wg = p.mfma ? pick_heads_per_wg_mfma(d, hq_per_kv)
@@ -152,19 +216,14 @@ DecodePlan plan_decode(int batch, int hq, int hq_per_kv, int d, int v_dtype, int
     return p;
   }
   const int tw = g_tuning[FDI4_TUNE_DECODE_TARGET_WAVES].load(std::memory_order_relaxed);
-  const int64_t target =
-      tw > 0 ? tw : (per_simd && p.waves == 4 ? kTargetWaves / 2 : kTargetWaves);
-  const int64_t per_split = (int64_t)batch * (hq / p.heads_per_wg) * p.waves;
-  const int s = (int)((target + per_split - 1) / per_split);
-  int smax = std::max(1, chunks / (p.waves * kMinChunksPerWave));
-  // Grouped heads (several q-heads per workgroup, more work per chunk) split
-  // down to one chunk per wave, up to eight splits (one merge round): in
-  // process A/B against four chunks per wave, one box: B1 Hkv8 Hq32 T1024
-  // 15.3 -> 12.0 us (8 splits against 2), B2 T2048 16.1 -> 13.8 (8 against
-  // 4), D64 B2 Hq64 T2048 14.9 -> 13.4, the shared-stream call of 8 x 256
-  // rows 19.1 -> 17.0; 16 and 32 splits were slower (B1 T4096 16.2 -> 22.3).
-  if (p.heads_per_wg > 1) smax = std::max(smax, std::min(chunks / p.waves, kMaxGroupedSplits));
-  p.splits = std::max(1, std::min(s, smax));
+  if (tw > 0) {
+    const int64_t per_split = streams * p.waves;
+    const int64_t s = (tw + per_split - 1) / per_split;
+    p.splits = (int)std::max<int64_t>(1, std::min<int64_t>(s, chunks / p.waves));
+    return p;
+  }
+  p.splits = pick_splits(streams, p.waves, chunks, d, v_dtype, p.mfma != 0,
+                         p.heads_per_wg > 1, hq_per_kv == 1, std::max(1, group_chunks));
   return p;
 }
 
@@ -522,7 +581,7 @@ int fdi4_decode_num_splits(int batch, int num_q_heads, const fdi4_paged_cache* c
       cache->num_kv_heads < 1 || num_q_heads % cache->num_kv_heads)
     return 1;
   return plan_decode(batch, num_q_heads, num_q_heads / cache->num_kv_heads, cache->head_dim,
-                     cache->v_dtype, chunks_per_seq(cache))
+                     cache->v_dtype, chunks_per_seq(cache), chunks_per_group(cache))
       .splits;
 }
 
@@ -576,7 +635,8 @@ int make_decode_args(const void* query, int q_dtype, int batch, int num_q_heads,
   if (cache->page_table && cache->pt_batch_stride < 0) return hipErrorInvalidValue;
   const int chunks = chunks_per_seq(cache);
   const DecodePlan plan = plan_decode(batch, num_q_heads, num_q_heads / cache->num_kv_heads,
-                                      cache->head_dim, cache->v_dtype, chunks);
+                                      cache->head_dim, cache->v_dtype, chunks,
+                                      chunks_per_group(cache));
   int splits = num_splits > 0 ? num_splits : plan.splits;
   splits = std::max(1, std::min(splits, std::max(chunks, 1)));
   a->q = query;
@@ -739,7 +799,7 @@ int fdi4_decode_step(const void* query, int query_dtype, int batch, int num_q_he
   // lies in one split): the append fuses into the decode (whose reads of a
   // group's staging rows take 32-bit byte offsets); with several splits the
   // merge follows it.
-  const int group_chunks = cache->pages_per_group * ceil_div(cache->page_rows, 16);
+  const int group_chunks = chunks_per_group(cache);
   const bool fused = !a.mfma && a.heads_per_wg == 1 && a.hq_per_kv == 1 &&
                      (a.num_splits == 1 || a.chunks_per_split % group_chunks == 0) &&
                      (int64_t)group_rows * st_row_stride * 4 <= INT32_MAX;
@@ -923,7 +983,7 @@ DenseLayout dense_layout(int B, int H, int D, int nb, int bs) {
     off += align_up((size_t)B * H * L.dp * sizeof(float));
   }
   // Every (sequence, head) attends the one shared page stream (kv-heads = 1).
-  L.splits = plan_decode(B, H, H, L.dp, FDI4_V_F32, nb * ceil_div(bs, 16)).splits;
+  L.splits = plan_decode(B, H, H, L.dp, FDI4_V_F32, nb * ceil_div(bs, 16), ceil_div(bs, 16)).splits;
   L.off_part = off;
   off += decode_ws_bytes(B, H, L.dp, L.splits);
   L.total = std::max<size_t>(off, kAlign);

@@ -129,7 +129,7 @@ decode_kernel(DecodeArgs a) {
   constexpr int NT = (WAVES + HW) * 64;
 
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int hk = fdiv(h, a.div_hpk);
+  const int hk = STEP ? h / a.hq_per_kv : fdiv(h, a.div_hpk);
   const int tid = threadIdx.x, lane = tid & 63;
   // The wave index is uniform across the wave; saying so keeps the chunk loop
   // counters in scalar registers and the page-table reads on the scalar unit.
@@ -185,7 +185,7 @@ decode_kernel(DecodeArgs a) {
   // copies are being written.
   const bool append = STEP && t_app >= 0;
   const int open_g = append ? t_app / a.step.group_rows : -1;
-  const int n_chunks = pages_of(a, T) * cpp;
+  const int n_chunks = pages_of<!STEP>(a, T) * cpp;
   const int c_begin = split * a.chunks_per_split;
   const int c_end = min(c_begin + a.chunks_per_split, n_chunks);
   // The split that holds the open group re-quantizes it (with several splits
@@ -265,7 +265,7 @@ decode_kernel(DecodeArgs a) {
   int c = 0;
   ChunkMeta cm{}, nm{};
   U32x4 sz[G::SZL];
-  auto meta_at = [&](int ci) { return chunk_meta(a, b, T, cpp, cidx(min(ci, wlen - 1))); };
+  auto meta_at = [&](int ci) { return chunk_meta<!STEP>(a, b, T, cpp, cidx(min(ci, wlen - 1))); };
   // Writes the wave's running partial (max logit, probability sum, weighted
   // values, each reduced over the wave) to LDS slot `slot` and restarts the
   // online softmax.

@@ -1,0 +1,45 @@
+"""The decode's split count over shapes (host arithmetic, no GPU): every split
+holds chunks, every wave of one its share, and the splits of short streams fill
+the 256 compute units once."""
+
+import os
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "int4-kv-cache-quantization-cuda-triton-pallas_amd")
+if PKG not in sys.path:
+    sys.path.insert(0, PKG)
+
+from flash_decode_int4 import capi  # noqa: E402
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("v_dtype", [capi.V_F32, capi.V_F16, capi.V_BF16])
+@pytest.mark.parametrize("kv_heads,rep", [(1, 1), (8, 1), (32, 1), (2, 2), (8, 4), (4, 8), (3, 3),
+                                          (1, 32)])
+def test_split_count(head_dim, v_dtype, kv_heads, rep):
+    lib = capi.load()
+    hq = kv_heads * rep
+    heads = {1: 1, 2: 2, 3: 1, 4: 4, 8: 8, 32: 8}[rep]
+    heads = min(heads, 4) if head_dim == 256 else heads
+    for batch in (1, 3, 17, 48, 300):
+        for rows in (1, 16, 250, 2048, 16000, 200000):
+            for page_rows in (1, 16, 256):
+                pages = -(-rows // page_rows)
+                cache = capi.PagedCache(max_pages=pages, page_rows=page_rows,
+                                        num_kv_heads=kv_heads, head_dim=head_dim,
+                                        v_dtype=v_dtype, pages_per_group=max(1, 256 // page_rows))
+                chunks = pages * -(-page_rows // 16)
+                s = lib.fdi4_decode_num_splits(batch, hq, cache)
+                assert 1 <= s <= 64
+                if s == 1:
+                    continue
+                per_split = -(-chunks // s)
+                assert -(-chunks // per_split) == s
+                assert per_split >= 4
+                # Short streams fill the compute units once (with two four-wave
+                # workgroups each, at most); long ones may take more, full rounds.
+                if batch * hq // heads <= 256 and rows <= 2048:
+                    assert batch * hq // heads * s <= 512

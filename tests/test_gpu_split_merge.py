@@ -1,0 +1,50 @@
+"""The split merge around its rounds of eight: any split count, splits that hold
+no rows, and values of empty splits that are never read."""
+
+import os
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+for p in (ROOT, os.path.join(ROOT, "int4-kv-cache-quantization-cuda-triton-pallas_amd")):
+    if p not in sys.path:
+        sys.path.insert(0, p)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("splits", [1, 2, 7, 8, 9, 16, 17, 64])
+def test_merge_of_given_partials(D, splits):
+    """Partials of known maxima, sums and values against float64; every third
+    split is empty (maximum -inf) and holds NaN values, one head has no rows."""
+    import torch
+    from flash_decode_int4._lib import load_binding
+    C = load_binding()
+    B, H = 2, 3
+    g = torch.Generator("cuda").manual_seed(D + splits)
+    n = B * H * splits
+    acc = torch.randn(B, H, splits, D, device="cuda", generator=g)
+    m = torch.randn(B, H, splits, device="cuda", generator=g).double() * 5
+    l = torch.rand(B, H, splits, device="cuda", generator=g).double() + 0.5
+    l = l.float().double()
+    empty = torch.zeros(B, H, splits, dtype=torch.bool, device="cuda")
+    empty[:, :, 1::3] = True
+    empty[1, 2] = True
+    m[empty] = -float("inf")
+    l[empty] = 0.0
+    acc[empty] = float("nan")
+    buf = torch.zeros(int(C.decode_partials_bytes(B, H, D, splits)), dtype=torch.uint8,
+                      device="cuda")
+    buf[:n * D * 4].view(torch.float32).copy_(acc.flatten())
+    off = (n * D * 4 + 255) // 256 * 256
+    buf[off:off + n * 16].view(torch.float64).copy_(torch.stack([m, l], -1).flatten())
+    out = C.merge_splits(buf, B, H, D, splits)
+    w = torch.where(empty, 0.0, torch.exp(m - m.amax(-1, keepdim=True).clamp(min=-1e300)))
+    want = (w[..., None] * torch.nan_to_num(acc.double())).sum(2)
+    want = want / (w * l).sum(-1, keepdim=True).clamp(min=1e-10)
+    # Each weight is a hardware exponential (1 ulp, argument rounded to 2^-24 of at
+    # most 60); sums of at most 64 float32 terms.
+    assert torch.equal(out[1, 2], torch.zeros_like(out[1, 2]))
+    assert (out - want).abs().max().item() < 2e-5 * want.abs().max().item()
