@@ -1,6 +1,5 @@
-"""The decode's split count over shapes (host arithmetic, no GPU): every split
-holds chunks, every wave of one its share, and the splits of short streams fill
-the 256 compute units once."""
+"""The decode's split count over shapes (host arithmetic, no GPU): bounded, and
+every split holds chunks, at least one for each wave of its workgroup."""
 
 import os
 import sys
@@ -22,8 +21,6 @@ from flash_decode_int4 import capi  # noqa: E402
 def test_split_count(head_dim, v_dtype, kv_heads, rep):
     lib = capi.load()
     hq = kv_heads * rep
-    heads = {1: 1, 2: 2, 3: 1, 4: 4, 8: 8, 32: 8}[rep]
-    heads = min(heads, 4) if head_dim == 256 else heads
     for batch in (1, 3, 17, 48, 300):
         for rows in (1, 16, 250, 2048, 16000, 200000):
             for page_rows in (1, 16, 256):
@@ -39,7 +36,3 @@ def test_split_count(head_dim, v_dtype, kv_heads, rep):
                 per_split = -(-chunks // s)
                 assert -(-chunks // per_split) == s
                 assert per_split >= 4
-                # Short streams fill the compute units once (with two four-wave
-                # workgroups each, at most); long ones may take more, full rounds.
-                if batch * hq // heads <= 256 and rows <= 2048:
-                    assert batch * hq // heads * s <= 512
