@@ -93,8 +93,9 @@ typedef struct fdi4_paged_cache {
  *                                  ones where registers allow)
  *   FDI4_TUNE_DECODE_HEADS_PER_WG  cap on q-heads per decode workgroup: 1
  *                                  (per-head kernel), 2, 4 or 8
- *   FDI4_TUNE_DECODE_TARGET_WAVES  resident waves the split count aims for
- *                                  (1 .. 1<<20)
+ *   FDI4_TUNE_DECODE_TARGET_WAVES  take the smallest split count that gives so
+ *                                  many waves (1 .. 1<<20) in place of the
+ *                                  estimated fastest
  *   FDI4_TUNE_FAKE_QUANT_SPLIT     channel slices per key row of
  *                                  fdi4_fake_quantize (1 .. 512)
  */
@@ -346,8 +347,9 @@ int fdi4_decode_paged_partials(const float* query, int batch, int num_q_heads,
  * is looked up, with hipGetSymbolAddress, on the first multi-split call on a
  * device: make that call once eagerly, outside any HIP graph capture, before
  * capturing the entry point; later calls only enqueue kernels and can be
- * captured). A call whose partials would
- * exceed the array returns hipErrorInvalidValue before any device work. The
+ * captured). A call whose num_splits needs more than the array returns
+ * hipErrorInvalidValue before any device work; an automatic count (num_splits
+ * <= 0) is cut down to what the array holds. The
  * caller still passes the inputs and the output. Calls that overlap on one GPU
  * (concurrent streams, or threads) share the array and race; serialize them.
  * No counterpart in the reference: for callers that cannot allocate device

@@ -922,6 +922,14 @@ int fdi4_decode_paged_noalloc(const float* query, int batch, int num_q_heads,
   int rc = make_decode_args(query, FDI4_K_F32, batch, num_q_heads, q_batch_stride,
                             q_head_stride, cache, num_splits, &a);
   if (rc != hipSuccess) return rc;
+  // An automatic count stays within the array (without this, plans of more
+  // splits than before would be refused).
+  if (num_splits <= 0) {
+    while (a.num_splits > 1 && decode_ws_bytes(batch, num_q_heads, cache->head_dim, a.num_splits) >
+                                   (size_t)FDI4_NOALLOC_SCRATCH_BYTES)
+      --a.num_splits;
+    a.chunks_per_split = std::max(1, ceil_div(chunks_per_seq(cache), a.num_splits));
+  }
   if (!out) return hipErrorInvalidValue;
   const int d = cache->head_dim;
   a.out = out;
