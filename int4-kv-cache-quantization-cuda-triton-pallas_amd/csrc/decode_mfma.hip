@@ -44,11 +44,11 @@
 // head's probability, widening, the LDS round trip of the probabilities and one
 // logit recombination per (row, column) cost more vector-unit time than that at
 // HG = 4 and twice as much at HG = 8. Measured against that form, per call with
-// the merge: B8 Hkv8 Hq32 T8192 bfloat16 37.6 -> 32.6 us (172 MB; the stream
-// itself now runs at 6.8 TB/s, the rest is the first 6 us and the last 3 of a
-// workgroup); D = 256 B4 Hkv4 Hq16 T4095 30.1 -> 19.9 us (against the vector
-// kernel); a B16 Hkv8 Hq64 float16 step of ragged lengths to 4096 56.8 -> 37.6 us;
-// B8 H32 over one float32 stream of 2048 rows 16.0 -> 13.9 us.
+// the merge: B8 Hkv8 Hq32 T8192 bfloat16 37.3 -> 31.3 us (172 MB; the stream
+// itself now runs at 6.8 TB/s, the rest is the first 6 us and the last 2 of a
+// workgroup and the merge); D = 256 B4 Hkv4 Hq16 T4095 30.0 -> 16.0 us (against
+// the vector kernel); a B16 Hkv8 Hq64 float16 step of ragged lengths to 4096
+// 56.7 -> 34.8 us; B8 H32 over one float32 stream of 2048 rows 16.0 -> 12.4 us.
 
 #include "decode_common.hpp"
 
