@@ -532,31 +532,35 @@ __global__ __launch_bounds__(64) void merge_kernel(const float* __restrict__ ws_
                                                    int splits, void* __restrict__ out,
                                                    int out_dtype, int64_t o_b, int64_t o_h) {
   constexpr int CH = D / 64, NB = 8;
-  struct alignas(4 * CH) Ch {
+  // No alignment beyond the element's: a caller's partials may start anywhere.
+  struct Ch {
     float v[CH];
+  };
+  struct Ml {
+    double m, l;
   };
   const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
   const int64_t p0 = ((int64_t)b * hq + h) * splits;
   const Ch* acc = reinterpret_cast<const Ch*>(ws_acc + p0 * D) + lane;
-  const double2* ml = reinterpret_cast<const double2*>(ws_ml + 2 * p0);
+  const Ml* ml = reinterpret_cast<const Ml*>(ws_ml + 2 * p0);
   double ms = -INFINITY;
   float l = 0.f;
   Ch o = {};
 #pragma unroll 1
   for (int s0 = 0; s0 < splits; s0 += NB) {
     const int mine = s0 + (lane & (NB - 1));
-    double2 x = ml[min(mine, splits - 1)];
+    Ml x = ml[min(mine, splits - 1)];
     Ch av[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) av[j] = acc[(int64_t)min(s0 + j, splits - 1) * 64];
-    if (mine >= splits) x = make_double2(-INFINITY, 0.0);
+    if (mine >= splits) x = Ml{-INFINITY, 0.0};
     // The running maximum (over eight lanes, the same in all), and what it does
     // to the sums of earlier rounds.
-    double mr = fmax(x.x, xchg<1>(x.x));
+    double mr = fmax(x.m, xchg<1>(x.m));
     mr = fmax(mr, xchg<2>(mr));
     mr = fmax(fmax(mr, xchg<4>(mr)), ms);
-    const bool live = x.x != -INFINITY;
-    const float e = live ? exp2_of(x.x - mr) : 0.f;
+    const bool live = x.m != -INFINITY;
+    const float e = live ? exp2_of(x.m - mr) : 0.f;
     if (s0 > 0 && ms != -INFINITY) {
       const float c = exp2_of(ms - mr);
       l *= c;
@@ -564,7 +568,7 @@ __global__ __launch_bounds__(64) void merge_kernel(const float* __restrict__ ws_
       for (int k = 0; k < CH; ++k) o.v[k] *= c;
     }
     ms = mr;
-    float lj = live ? e * (float)x.y : 0.f;
+    float lj = live ? e * (float)x.l : 0.f;
     lj += xchg<1>(lj);
     lj += xchg<2>(lj);
     l += lj + xchg<4>(lj);

@@ -48,3 +48,23 @@ def test_merge_of_given_partials(D, splits):
     # most 60); sums of at most 64 float32 terms.
     assert torch.equal(out[1, 2], torch.zeros_like(out[1, 2]))
     assert (out - want).abs().max().item() < 2e-5 * want.abs().max().item()
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_merge_of_partials_at_any_alignment(D):
+    """fdi4_merge_splits takes partials that start at any element."""
+    import torch
+    from flash_decode_int4 import capi
+    lib = capi.load()
+    B, H, S = 2, 2, 5
+    g = torch.Generator("cuda").manual_seed(D)
+    acc = torch.randn(B * H * S * D + 3, device="cuda", generator=g)
+    ml = torch.rand(B * H * S * 2 + 1, device="cuda", generator=g, dtype=torch.float64) + 0.5
+    outs = []
+    for a, m in ((acc[3:], ml[1:]), (acc[3:].clone(), ml[1:].clone())):
+        out = torch.empty(B, H, D, device="cuda")
+        capi.check(lib.fdi4_merge_splits(a.data_ptr(), m.data_ptr(), B, H, D, S, out.data_ptr(),
+                                         out.stride(0), out.stride(1),
+                                         torch.cuda.current_stream().cuda_stream), "merge")
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
