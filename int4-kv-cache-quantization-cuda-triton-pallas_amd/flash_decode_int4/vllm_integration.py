@@ -390,6 +390,10 @@ class INT4PagedSequenceCache:
         import torch
         lens = np.asarray(seq_lens.cpu() if hasattr(seq_lens, "cpu") else seq_lens, np.int64)
         lens = lens.reshape(-1)
+        if torch.cuda.is_current_stream_capturing():
+            # The lengths and pages of this call are host data; a replay would
+            # read their transfer buffer again.
+            raise RuntimeError("prefill() cannot be captured into a graph")
         self._check_prefill(k, v, lens)
         B = k.shape[0]
         self._sync_if_stepped()

@@ -127,3 +127,21 @@ def test_prefill_from_two_streams():
     torch.cuda.synchronize()
     for c, n in zip(caches, (595, 232)):
         _check(c, k, k, [n, 600 - n // 2])
+
+
+def test_prefill_is_refused_under_capture():
+    import torch
+    from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
+    c = INT4PagedSequenceCache(8, 2, 64, 2, 64, 16, 64, "float32")
+    k = torch.randn(2, 2, 40, 64, device="cuda")
+    c.prefill(k, k.clone(), [40, 3])
+    x = torch.zeros(4, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x += 1
+        with pytest.raises(RuntimeError, match="captured"):
+            c.prefill(k, k, [5, 6])
+    graph.replay()
+    torch.cuda.synchronize()
+    assert x.tolist() == [1.0] * 4
+    _check(c, k, k, [40, 3])
