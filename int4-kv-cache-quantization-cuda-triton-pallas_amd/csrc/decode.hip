@@ -514,8 +514,10 @@ decode_kernel(DecodeArgs a) {
 }
 
 // Log-sum-exp merge of the split partials: grid (Hq, B), one wave, D / 64
-// channels a lane. Split s adds nothing when its maximum is -inf (no rows); the
-// others add exp(m_s - max) times their values and sums. The partials of eight
+// channels a lane. A split of no rows (maximum -inf, sum 0) adds nothing; the
+// others add exp(m_s - max) times their values and sums. (A maximum passes NaN
+// over, so a split whose logits are NaN has the maximum -inf too, but a NaN sum,
+// which makes the result NaN.) The partials of eight
 // splits are in flight at a time; lane j holds split j's maximum and sum and
 // computes its weight once, and the lanes take the weights as scalars.
 //
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(64) void merge_kernel(const float* __restrict__ ws_
     double mr = fmax(x.m, xchg<1>(x.m));
     mr = fmax(mr, xchg<2>(mr));
     mr = fmax(fmax(mr, xchg<4>(mr)), ms);
-    const bool live = x.m != -INFINITY;
+    const bool live = !(x.m == -INFINITY && x.l == 0.0);
     const float e = live ? exp2_of(x.m - mr) : 0.f;
     if (s0 > 0 && ms != -INFINITY) {
       const float c = exp2_of(ms - mr);

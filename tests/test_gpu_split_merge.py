@@ -68,3 +68,37 @@ def test_merge_of_partials_at_any_alignment(D):
                                          torch.cuda.current_stream().cuda_stream), "merge")
         outs.append(out)
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("bad", ["nan", "inf", "-inf"])
+@pytest.mark.parametrize("splits", [1, 2, 9])
+@pytest.mark.parametrize("rep,vector,vdtype", [(1, 0, "float32"), (4, 0, "float32"),
+                                               (4, 0, "float16"), (4, 1, "float32")])
+def test_non_finite_query(rep, vector, vdtype, splits, bad):
+    """A NaN or infinite query element makes its head's output NaN in every kernel
+    and at every split count (a split of NaN logits has the maximum of an empty
+    one, -inf, but not its sum); the other heads keep theirs."""
+    import torch
+    from flash_decode_int4 import capi, ops
+    B, H, D, T = 2, 2, 128, 700
+    g = torch.Generator("cuda").manual_seed(splits)
+    cols = -(-T // 16)
+    pt = torch.randperm(B * cols, device="cuda", generator=g).to(torch.int32).view(B, cols)
+    sl = torch.tensor([T, 130], dtype=torch.int32, device="cuda")
+    kp = torch.zeros(B * cols, H, 16, D // 2, dtype=torch.uint8, device="cuda")
+    s = torch.zeros(B, H, -(-T // 128), D, device="cuda")
+    z = torch.zeros_like(s)
+    ops.quantize_int4_paged(torch.randn(B, H, T, D, device="cuda", generator=g), sl, pt, kp, s, z)
+    v = torch.randn(B * cols, H, 16, D, device="cuda", generator=g).to(getattr(torch, vdtype))
+    q = torch.randn(B, H * rep, D, device="cuda", generator=g) * (2.0 / D ** 0.5)
+    qb = q.clone()
+    qb[0, 1, 3] = float(bad)
+    qb[1, 0, D - 1] = float(bad)
+    with capi.tuning(decode_vector_only=vector):
+        good = ops.flash_decode_paged(q, kp, v, s, z, pt, sl, num_splits=splits)
+        out = ops.flash_decode_paged(qb, kp, v, s, z, pt, sl, num_splits=splits)
+    hit = torch.zeros(B, H * rep, dtype=torch.bool, device="cuda")
+    hit[0, 1] = hit[1, 0] = True
+    assert torch.isnan(out[hit]).all()
+    # The same sums, or (float16) those of the float32 products: 700 terms.
+    assert (out[~hit] - good[~hit]).abs().max().item() < 2e-6
