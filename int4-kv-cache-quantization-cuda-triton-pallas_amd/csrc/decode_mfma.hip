@@ -30,9 +30,17 @@
 //      4g .. 4g+3; byte permutes pair the rows, and each 16x16x16 product adds
 //      four rows a lane group to the output of 16 channels x 16 columns. A
 //      float32 probability is the exact sum of three 8-bit (bfloat16) or
-//      11-bit (float16, scaled by 2^15) terms, which sit in different columns
-//      of the head (HG = 8: two columns, so two products), so the products are
-//      exact, their sums are float32, and one instruction does all terms. Only the final output adds the columns up.
+//      11-bit (float16) terms, which sit in different columns of the head
+//      (HG = 8: the first term in one column, the others in the second, in two
+//      products), so the products are exact, their sums are float32, and one
+//      instruction does all terms. Only the final output adds the columns up.
+//      float16 has 40 binades for the terms: they are scaled by 2^15 (the first)
+//      and 2^25 (the others), which holds every bit of a probability down to
+//      2^-26. A chunk with a smaller one (a row 18 below the wave's maximum in
+//      the logit) takes the float32 products below, in the first column: with
+//      logits of standard deviation 2 none does; where every chunk does (12), a
+//      B8 Hkv8 Hq32 T8192 decode takes 41 us in place of 32, B16 Hkv8 Hq64 ragged
+//      to 4096 45 in place of 27.
 //      A non-finite value times an empty term is NaN where the float32 product
 //      is infinite: a wave that ends with a NaN runs its range again with the
 //      float32 products below.
@@ -211,9 +219,13 @@ template <int D, int VDT, int WAVES, int HG>
 __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   using G = MfmaGeo<D, VDT, HG>;
   constexpr int NT = WAVES * 64, CPH = G::CPH, RN = G::RN;
-  // float16 terms of a probability are those of p * 2^15 (still finite), so
-  // that they keep 24 bits down to p = 2^-15 and 2^-39 below.
-  constexpr float kPScale = VDT == kVF16 ? 32768.f : 1.f;
+  // float16 terms of a probability: the first is that of p * 2^15 (p <= 1, so it
+  // is finite), the others those of the remainder (below 2^-10 p) times 2^25. The
+  // last bit of p is at least 2^-49 from p = 2^-26 up, so every term is a multiple
+  // of float16's smallest number.
+  constexpr float kPScale = VDT == kVF16 ? 0x1p15f : 1.f;
+  constexpr float kRestScale = VDT == kVF16 ? 0x1p10f : 1.f;   // of the others, beyond it
+  constexpr float kLeastP = 0x1p-26f * kPScale;
 
   const int split = blockIdx.x, b = blockIdx.z;
   const int h0 = blockIdx.y * HG;           // first q-head of this workgroup
@@ -508,13 +520,8 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
         v4f t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float v;
-          if constexpr (VDT == kVF32) v = u2f(f.v[i][u][j]);
-          else if constexpr (VDT == kVF16)
-            v = (float)__builtin_bit_cast(_Float16,
-                                          (unsigned short)(f.v[i][u][j / 2] >> (16 * (j & 1))));
-          else v = u2f(j & 1 ? f.v[i][u][j / 2] & 0xFFFF0000u : f.v[i][u][j / 2] << 16);
-          t[i / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, x[i], t[i / 2], 0, 0, 0);
+          t[i / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(u2f(f.v[i][u][j]), x[i], t[i / 2],
+                                                          0, 0, 0);
         }
         v4f& o = acc[u * G::CPP + j];
 #pragma unroll
@@ -522,30 +529,53 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
       }
   };
 
+  // The same with 16-bit values, for the rare chunks whose probabilities or
+  // values the 16-bit products below would not hold: products added to the
+  // accumulators one after the other, which takes no registers for chunk sums
+  // (those would cost every chunk a wave of occupancy).
+  auto value_wide = [&](const Buf& f, const float* x) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < G::NP; ++u)
+#pragma unroll
+      for (int j = 0; j < G::CPP; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const unsigned w = f.v[i][u][j / 2];
+          float v;
+          if constexpr (VDT == kVF16)
+            v = (float)__builtin_bit_cast(_Float16, (unsigned short)(w >> (16 * (j & 1))));
+          else
+            v = u2f(j & 1 ? w & 0xFFFF0000u : w << 16);
+          v4f& t = acc[u * G::CPP + j];
+          t = __builtin_amdgcn_mfma_f32_16x16x4f32(v, x[i], t, 0, 0, 0);
+        }
+  };
+
   // Upper bits of a probability that one 16-bit term holds.
   constexpr unsigned kTerm = VDT == kVF16 ? 0xFFFFE000u : 0xFFFF0000u;
-  // Two terms packed as the 16-bit type (their lower bits are zero or, below
-  // the smallest, dropped).
+  // Two terms packed as the 16-bit type: the bits below a term's are dropped.
   auto pack2 = [&](float lo, float hi) __attribute__((always_inline)) -> unsigned {
     if constexpr (VDT == kVF16)
       return __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(lo, hi));
     else
       return __builtin_amdgcn_perm(f2u(hi), f2u(lo), 0x07060302u);
   };
-  const unsigned term1 = col >= 1 ? kTerm : 0u, term2 = col >= 2 ? kTerm : 0u;
+  // Bits of a probability that go to earlier columns, first term and second; at
+  // HG = 8 what the second product of column 0 leaves out is everything.
+  const unsigned term1 = col >= 1 ? kTerm : 0u;
+  const unsigned term2 = CPH == 2 ? (col == 0 ? ~0u : kTerm) : (col >= 2 ? kTerm : 0u);
+  const float rest = col >= 1 ? kRestScale : 1.f;
 
   // 16-bit products of the values with the terms of the probabilities x.
   auto value_16 = [&](const Buf& f, const float* x) __attribute__((always_inline)) {
     unsigned bt[4];
     if constexpr (CPH == 2) {
-      // Column 0: first, then second term; column 1: third, then nothing.
+      // Column 0: first term, then nothing; column 1: second, then third term.
       float ta[4], tb[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float r1 = x[i] - u2f(f2u(x[i]) & kTerm);
-        const float r2 = r1 - u2f(f2u(r1) & kTerm);
-        ta[i] = odd ? r2 : x[i];
-        tb[i] = odd ? 0.f : r1;
+        ta[i] = x[i] - u2f(f2u(x[i]) & term1);
+        tb[i] = ta[i] - u2f(f2u(ta[i]) & term2);
       }
       bt[0] = pack2(ta[0], ta[1]);
       bt[1] = pack2(ta[2], ta[3]);
@@ -553,6 +583,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
       bt[3] = pack2(tb[2], tb[3]);
     } else {
       // Column c: term c (columns 3 and beyond repeat term 2 and are dropped).
+      // (Masks keep leading bits, so the columns' scale may come before them.)
       float t[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -635,11 +666,33 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
       x[2] = u2f(dpp<0xA0>(f2u(p[RN - 1])));
       x[3] = u2f(dpp<0xF5>(f2u(p[RN - 1])));
     }
+    if constexpr (VDT == kVF16) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] *= rest;
+    }
     if constexpr (VDT == kVF32) {
       value_f32(f, x, corr);
+    } else if (wide) {
+      value_wide(f, x);
     } else {
-      if (wide) value_f32(f, x, 1.f);
-      else value_16(f, x);
+      if constexpr (VDT == kVF16) {
+        bool small = false;   // 0 < p < kLeastP
+#pragma unroll
+        for (int k = 0; k < RN; ++k) small |= f2u(p[k]) - 1u < f2u(kLeastP) - 1u;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(small) != 0, 0)) {
+          // The float32 products, in column 0, and then 16-bit products of
+          // nothing: with those in the other branch the accumulators would be
+          // copied where the branches meet, in every chunk.
+          float x0[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x0[i] = col == 0 ? x[i] : 0.f;
+            x[i] = 0.f;
+          }
+          value_wide(f, x0);
+        }
+      }
+      value_16(f, x);
     }
   };
 
@@ -739,13 +792,14 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
         p = chunk_next(p, cpp, ppg);
       }
     }
-    // The terms' columns add up (small terms first).
+    // The terms' columns add up, each taken back by its scale.
+    const float back = col == 0 ? 1.f / kPScale : 1.f / (kPScale * kRestScale);
 #pragma unroll
     for (int t = 0; t < G::NA; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float x = col < cols ? acc[t][i] : 0.f;
-        acc[t][i] = allreduce_sum<1, (CPH >= 4 ? 4 : 2)>(x) * (1.f / kPScale);
+        const float x = col < cols ? acc[t][i] * back : 0.f;
+        acc[t][i] = allreduce_sum<1, (CPH >= 4 ? 4 : 2)>(x);
       }
   }
 

@@ -71,3 +71,48 @@ def test_huge_logits(D, rep, vdtype, scale):
     with capi.tuning(decode_heads_per_wg=1):
         b = ops.flash_decode_paged(q * scale, kp, v, s, z, pt, sl)
     assert (a - b).abs().max().item() < 2e-6
+
+
+def _exact(q, kp, v, s, z, pt, sl, rep, group_rows=128):
+    """float64 attention over the valid rows alone."""
+    import torch
+    B, Hq, D = q.shape
+    H = kp.shape[1]
+    out = []
+    for b in range(B):
+        n = int(sl[b])
+        pages = pt[b].long()
+        k = kp[pages].permute(1, 0, 2, 3).reshape(H, -1, D // 2)[:, :n]
+        k = torch.stack([k & 15, k >> 4], -1).reshape(H, n, D).double()
+        k = ((k - z[b].double().repeat_interleave(group_rows, 1)[:, :n])
+             * s[b].double().repeat_interleave(group_rows, 1)[:, :n])
+        x = v[pages].permute(1, 0, 2, 3).reshape(H, -1, D)[:, :n].double()
+        w = torch.softmax(torch.bmm(q[b].double().view(H, rep, D),
+                                    k.transpose(1, 2).contiguous()), -1)
+        # (a sum of products per channel: a zero weight times an infinity is NaN)
+        out.append((w[..., None] * x[:, None]).sum(2).reshape(Hq, D))
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("D,rep,vdtype", SHAPES)
+@pytest.mark.parametrize("gap", [8.0, 16.0, 24.0, 40.0, 60.0])
+def test_dominant_row_of_value_zero(D, rep, vdtype, gap):
+    """A row whose logit lies `gap` above the others' and whose value is zero (an
+    attention sink): the output is the sum of probabilities of exp(-gap), which
+    keep their 24 bits."""
+    import torch
+    ops, q, kp, v, s, z, pt, sl = _inputs(D, rep, vdtype, [1000, 77])
+    B, Hq, _ = q.shape
+    for b in range(B):
+        page = pt[b, 0].item()
+        v[page, :, 0] = 0
+        k = torch.stack([kp[page, :, 0] & 15, kp[page, :, 0] >> 4], -1).reshape(2, D)
+        k = (k - z[b, :, 0]) * s[b, :, 0]
+        k = k * (gap / (k * k).sum(-1, keepdim=True))
+        q[b] = (0.3 * q[b].view(2, rep, D) + k[:, None]).view(Hq, D)
+    a = ops.flash_decode_paged(q, kp, v, s, z, pt, sl, num_splits=1)
+    b = _exact(q, kp, v, s, z, pt, sl, rep)
+    # Each weight is exp2 of an argument rounded to 24 bits: 2^-24 of up to
+    # gap / ln 2 and a unit in the last place, and as much for the merge of waves.
+    bound = 2.0 ** -24 * (2 * gap + 8)
+    assert ((a - b).norm() / b.norm()).item() < bound
