@@ -630,14 +630,16 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     mc = max_raw(mc, xchg<1>(mc));
     if constexpr (CPH >= 4) mc = max_raw(mc, xchg<2>(mc));
     mc = groups_max(mc);
-    // The shift: the float32 maximum of the rounded logits, raised by two of
-    // its ulps so that no probability exceeds 1 -- or, where two ulps are more
-    // than a quarter, the double maximum itself.
-    double mx = __builtin_fma(__builtin_fabs((double)mc), 0x1p-22, (double)mc);
-    if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(mc) < 0x1p20f))) {
+    // The shift: the maximum of the rounded logits, brought up to a whole number,
+    // so that every factor between shifts (chunks, waves, splits) is an exact
+    // power of two -- from 2^20 up, where a float32 logit is off by 1/16 and more,
+    // the double maximum. A probability exceeds 1 by a factor 2^(1/16) at most.
+    double mx = __builtin_ceil((double)mc);
+    if (__builtin_expect(
+            __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(mc) < 0x1p20f)) != 0, 0)) {
       mx = lg[0];
       if constexpr (RN > 1) mx = fmax(mx, lg[RN - 1]);
-      mx = allreduce_max<16, 64>(allreduce_max<1, (CPH >= 4 ? 4 : 2)>(mx));
+      mx = __builtin_ceil(allreduce_max<16, 64>(allreduce_max<1, (CPH >= 4 ? 4 : 2)>(mx)));
     }
     const double m_new = max_raw(m_run, mx);
     const float corr = __builtin_amdgcn_exp2f((float)(m_run - m_new));
@@ -835,31 +837,48 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     double ms = -INFINITY;
 #pragma unroll
     for (int i = 0; i < WAVES; ++i) ms = fmax(ms, m_s[i][h]);
-    float o[4] = {0.f, 0.f, 0.f, 0.f}, l = 0.f;
+    // Weighted waves, then their sum as a tree (the weights are powers of two, so
+    // only its additions round; as one chain they were the larger part of a short
+    // sequence's error).
+    float l[WAVES], o[WAVES][4];
 #pragma unroll
     for (int i = 0; i < WAVES; ++i) {
       const float e =
           (m_s[i][h] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((float)(m_s[i][h] - ms));
-      l = __builtin_fmaf(e, l_s[i][h], l);
       const float4 x = *reinterpret_cast<const float4*>(
           reinterpret_cast<const float*>(wave_s[i]) + idx);
-      o[0] = __builtin_fmaf(e, x.x, o[0]);
-      o[1] = __builtin_fmaf(e, x.y, o[1]);
-      o[2] = __builtin_fmaf(e, x.z, o[2]);
-      o[3] = __builtin_fmaf(e, x.w, o[3]);
+      const float xs[4] = {x.x, x.y, x.z, x.w};
+      if (i & 1) {
+        l[i / 2] = __builtin_fmaf(e, l_s[i][h], l[i / 2]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[i / 2][k] = __builtin_fmaf(e, xs[k], o[i / 2][k]);
+      } else {
+        l[i / 2] = e * l_s[i][h];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[i / 2][k] = e * xs[k];
+      }
     }
+#pragma unroll
+    for (int n = WAVES / 4; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        l[i] = l[2 * i] + l[2 * i + 1];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[i][k] = o[2 * i][k] + o[2 * i + 1][k];
+      }
     const int hq = h0 + h;
     if (a.final_out) {
-      const float r = fmaxf(l, 1e-10f);
+      const float r = fmaxf(l[0], 1e-10f);
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        store_elem(a.out, (int64_t)b * a.o_b + (int64_t)hq * a.o_h + d + k, a.out_dtype, o[k] / r);
+        store_elem(a.out, (int64_t)b * a.o_b + (int64_t)hq * a.o_h + d + k, a.out_dtype,
+                   o[0][k] / r);
     } else {
       const int64_t pi = ((int64_t)b * a.num_q_heads + hq) * a.num_splits + split;
-      *reinterpret_cast<float4*>(a.ws_acc + pi * D + d) = make_float4(o[0], o[1], o[2], o[3]);
+      *reinterpret_cast<float4*>(a.ws_acc + pi * D + d) = make_float4(o[0][0], o[0][1], o[0][2], o[0][3]);
       if (d == 0) {
         a.ws_ml[2 * pi] = ms * 0.6931471805599453;   // natural log units
-        a.ws_ml[2 * pi + 1] = (double)l;
+        a.ws_ml[2 * pi + 1] = (double)l[0];
       }
     }
   }

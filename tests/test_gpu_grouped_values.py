@@ -20,10 +20,10 @@ SHAPES = [(64, 2, "float16"), (64, 8, "bfloat16"), (128, 2, "bfloat16"), (128, 4
           (256, 4, "float32")]
 
 
-def _inputs(D, rep, vdtype, lens):
+def _inputs(D, rep, vdtype, lens, seed=0):
     import torch
     from flash_decode_int4 import ops
-    g = torch.Generator("cuda").manual_seed(D + rep)
+    g = torch.Generator("cuda").manual_seed(D + rep + 1000 * seed)
     B, H, T = len(lens), 2, max(lens)
     cols = -(-T // 16)
     pt = torch.randperm(B * cols, device="cuda", generator=g).to(torch.int32).view(B, cols)
@@ -89,8 +89,9 @@ def _exact(q, kp, v, s, z, pt, sl, rep, group_rows=128):
         x = v[pages].permute(1, 0, 2, 3).reshape(H, -1, D)[:, :n].double()
         w = torch.softmax(torch.bmm(q[b].double().view(H, rep, D),
                                     k.transpose(1, 2).contiguous()), -1)
-        # (a sum of products per channel: a zero weight times an infinity is NaN)
-        out.append((w[..., None] * x[:, None]).sum(2).reshape(Hq, D))
+        # (per head: an infinite value spoils no more than its own channel)
+        out.append(torch.stack([(w[h, j][:, None] * x[h]).sum(0)
+                                for h in range(H) for j in range(rep)]))
     return torch.stack(out)
 
 
@@ -116,3 +117,21 @@ def test_dominant_row_of_value_zero(D, rep, vdtype, gap):
     # gap / ln 2 and a unit in the last place, and as much for the merge of waves.
     bound = 2.0 ** -24 * (2 * gap + 8)
     assert ((a - b).norm() / b.norm()).item() < bound
+
+
+@pytest.mark.parametrize("D,rep,vdtype", [(64, 2, "float16"), (64, 8, "bfloat16"),
+                                          (128, 2, "float16"), (128, 8, "float16"),
+                                          (128, 4, "bfloat16"), (64, 2, "float32")])
+def test_error_against_float64(D, rep, vdtype):
+    """The relative error of the automatic plan (many splits here), over twelve
+    seeds, below that of float32 FMAs of each row in eight splits: 1.6e-7 to
+    1.7e-7 at these sizes."""
+    import torch
+    a = n = 0.0
+    for seed in range(12):
+        ops, q, kp, v, s, z, pt, sl = _inputs(D, rep, vdtype, [8192, 8192], seed)
+        e = _exact(q, kp, v, s, z, pt, sl, rep)
+        o = ops.flash_decode_paged(q, kp, v, s, z, pt, sl)
+        a += ((o - e) ** 2).sum().item()
+        n += (e ** 2).sum().item()
+    assert (a / n) ** 0.5 < 1.5e-7
