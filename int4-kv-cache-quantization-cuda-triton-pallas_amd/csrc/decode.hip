@@ -403,6 +403,13 @@ decode_kernel(DecodeArgs a) {
         }
       }
     }
+    // Lanes past the valid rows hold the last valid row; zeros in its place, lest
+    // an infinity there times their probability 0 be NaN.
+    if (cm.nval < 16) {
+#pragma unroll
+      for (int i = 0; i < G::VLD; ++i)
+        if (i * G::RPL + vrow >= cm.nval) cv[i] = U32x4{0, 0, 0, 0};
+    }
 #pragma unroll
     for (int k = 0; k < G::VCL; ++k) acc[k] *= corr;
 #pragma unroll

@@ -162,7 +162,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_gqa_kernel(DecodeArgs a) {
   ChunkMeta cm, nm;
   U32x4 sz[G::SZL];
   auto meta_at = [&](int ci) { return chunk_meta(a, b, T, cpp, min(ci, wc1 - 1)); };
-  auto step = [&](const KVec<1>* ck, const U32x4* cv, KVec<1>* nk, U32x4* nv) -> bool {
+  auto step = [&](const KVec<1>* ck, U32x4* cv, KVec<1>* nk, U32x4* nv) -> bool {
     if (cm.group != cur_group) {
       float* szw = sz_s[w];
 #pragma unroll
@@ -255,11 +255,16 @@ __global__ __launch_bounds__(WAVES * 64) void decode_gqa_kernel(DecodeArgs a) {
 #pragma unroll
         for (int k = 0; k < G::VCL; ++k) acc[h][k] *= corr[h];
       }
+      // Rows past the valid count hold probability 0 (their logits are -inf) and
+      // a copy of a valid row: zeros in its place, lest an infinity there be NaN.
+      if (cm.nval < 16) {
+#pragma unroll
+        for (int i = 0; i < G::VLD; ++i)
+          if (i * G::RPL + vrow >= cm.nval) cv[i] = U32x4{0, 0, 0, 0};
+      }
 #pragma unroll
       for (int i = 0; i < G::VLD; ++i) {
         const int r = i * G::RPL + vrow;
-        // Rows past the valid count hold probability 0 (their logits are
-        // -inf), and their value registers hold a copy of a valid row.
         const HeadP<HG> pr = p_s[w][r];
         float vf[G::VCL];
         widen_values<VDT>(cv[i], vf);

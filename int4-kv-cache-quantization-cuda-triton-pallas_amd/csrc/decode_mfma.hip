@@ -618,7 +618,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
 
   // Consume one chunk of nval > 0 rows. wide: float32 products also for 16-bit
   // values.
-  auto consume = [&](const Buf& f, int nval, bool wide) __attribute__((always_inline)) {
+  auto consume = [&](Buf& f, int nval, bool wide) __attribute__((always_inline)) {
     double lg[RN];
     logits(f, lg);
     float mc = -INFINITY;
@@ -672,6 +672,19 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[i] *= rest;
     }
+    // Rows past the valid ones hold the last valid row: zeros in its place, lest
+    // an infinity there times their probability 0 be NaN. (The 16-bit products
+    // leave such a NaN to the run with float32 ones.)
+    if ((VDT == kVF32 || wide) && nval < 16) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned keep = 4 * grp + i < nval ? ~0u : 0u;
+#pragma unroll
+        for (int u = 0; u < G::NP; ++u)
+#pragma unroll
+          for (int k = 0; k < G::PB / 4; ++k) f.v[i][u][k] &= keep;
+      }
+    }
     if constexpr (VDT == kVF32) {
       value_f32(f, x, corr);
     } else if (wide) {
@@ -713,7 +726,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     if (ci < wc1) np = chunk_next(np, cpp, ppg);
     return pos_meta(a, pgm, T, np);
   };
-  auto step = [&](const Buf& f, Buf& nf) __attribute__((always_inline)) -> bool {
+  auto step = [&](Buf& f, Buf& nf) __attribute__((always_inline)) -> bool {
     if (mq[0].group != cur_group) {
       rebuild(sz);
       cur_group = mq[0].group;

@@ -95,6 +95,28 @@ def _exact(q, kp, v, s, z, pt, sl, rep, group_rows=128):
     return torch.stack(out)
 
 
+@pytest.mark.parametrize("D,rep,vdtype", SHAPES + [(64, 1, "float32"), (128, 1, "bfloat16"),
+                                                   (256, 1, "float16")])
+@pytest.mark.parametrize("vector", [0, 1])
+def test_infinite_value_in_the_last_row(D, rep, vdtype, vector):
+    """Lanes past the valid rows of a chunk hold the last valid row: an infinity
+    there must come out as the infinity that row alone gives, whatever the length
+    modulo 16."""
+    import torch
+    from flash_decode_int4 import capi
+    ops, q, kp, v, s, z, pt, sl = _inputs(D, rep, vdtype, [700, 133, 1, 96])
+    for b, n in enumerate([700, 133, 1, 96]):
+        v[pt[b, (n - 1) // 16].item(), b % 2, (n - 1) % 16, 3 + b] = (-1) ** b * float("inf")
+    with capi.tuning(decode_vector_only=vector):
+        a = ops.flash_decode_paged(q, kp, v, s, z, pt, sl)
+    b = _exact(q, kp, v, s, z, pt, sl, rep)
+    assert torch.isinf(b).sum().item() == 4 * rep
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    assert torch.equal(a[torch.isinf(b)].double(), b[torch.isinf(b)])
+    f = torch.isfinite(b)
+    assert (a[f] - b[f]).abs().max().item() < 2e-6
+
+
 @pytest.mark.parametrize("D,rep,vdtype", SHAPES)
 @pytest.mark.parametrize("gap", [8.0, 16.0, 24.0, 40.0, 60.0])
 def test_dominant_row_of_value_zero(D, rep, vdtype, gap):
