@@ -397,20 +397,16 @@ class INT4PagedSequenceCache:
         self._check_prefill(k, v, lens)
         B = k.shape[0]
         self._sync_if_stepped()
-        for b in range(B):
-            self._release(b)
-        # _check_prefill has seen to it that the pages exist: they leave the free
-        # list in one slice (the order successive pops would give).
+        # The pages as B releases and then successive pops would give them: the
+        # slots' own, then the free list's last. (_check_prefill has seen to it that
+        # there are enough.)
         need = (lens + self.page_rows - 1) // self.page_rows
         ends = np.cumsum(need).tolist()
         total = ends[-1] if B else 0
-        at = len(self._free) - total
-        taken = self._free[at:][::-1]
-        del self._free[at:]
-        for b, (n, end) in enumerate(zip(need.tolist(), ends)):
-            self._pages[b] = taken[end - n:end]
-        self._mapped[:B] = need * self.page_rows
-        self._lens[:B] = lens
+        back = [p for b in range(B) for p in reversed(self._pages[b])]
+        own, kept = back[max(0, len(back) - total):], back[:max(0, len(back) - total)]
+        cut = len(self._free) - (total - len(own))
+        taken = own[::-1] + self._free[cut:][::-1]
         # One launch: the sequences' page-table rows and lengths go along with
         # it, and the kernel writes them to the device arrays.
         table = np.zeros((B, int(need.max(initial=0))), np.int32)
@@ -422,6 +418,13 @@ class INT4PagedSequenceCache:
                                      torch.from_numpy(table), self.k_stage, self.k_pages,
                                      self.v_pages, self.k_scale, self.k_zp, self.page_table,
                                      self.seq_lens, self.group_rows)
+        # Launched: the host's lists follow. A call that failed before (the copy of
+        # v, the transfer buffers, the launch) leaves them and the device as they were.
+        self._free[cut:] = kept
+        for b, (n, end) in enumerate(zip(need.tolist(), ends)):
+            self._pages[b] = taken[end - n:end]
+        self._mapped[:B] = need * self.page_rows
+        self._lens[:B] = lens
 
     def append(self, k_new, v_new) -> None:
         """Append one token to each of sequences 0..B-1: k_new float32 and v_new

@@ -145,3 +145,41 @@ def test_prefill_is_refused_under_capture():
     torch.cuda.synchronize()
     assert x.tolist() == [1.0] * 4
     _check(c, k, k, [40, 3])
+
+
+@pytest.mark.parametrize("fails", ["launch", "clone"])
+def test_failed_prefill_changes_nothing(fails, monkeypatch):
+    """A call that fails after its arguments were accepted (the copy of unaligned
+    values, the launch) leaves the host's lists and the device's table and
+    lengths as they were, and a later call works."""
+    import torch
+    from flash_decode_int4 import vllm_integration as vi
+    c = vi.INT4PagedSequenceCache(24, 2, 64, 3, 160, 16, 64, "float16")
+    g = torch.Generator("cuda").manual_seed(2)
+    k = torch.randn(2, 2, 150, 64, device="cuda", generator=g)
+    v = torch.randn(2, 2, 64, 150, device="cuda", generator=g).half().transpose(2, 3)
+    c.prefill(k, v, [150, 33])
+
+    def state():
+        return (list(c._free), [list(p) for p in c._pages], c._mapped.tolist(),
+                c.lengths().tolist(), c.page_table.tolist(), c.seq_lens.tolist())
+
+    before = state()
+
+    class Failing:
+        def __getattr__(self, name):
+            def fail(*args, **kwargs):
+                raise RuntimeError("no memory")
+            return fail
+
+    with monkeypatch.context() as m:
+        if fails == "launch":
+            m.setattr(vi, "load_binding", lambda: Failing())
+        else:
+            m.setattr(torch.Tensor, "clone", Failing().clone)
+        with pytest.raises(RuntimeError, match="no memory"):
+            c.prefill(k, v, [100, 140])
+    assert state() == before
+    _check(c, k, v, [150, 33])
+    c.prefill(k, v, [100, 140])
+    _check(c, k, v, [100, 140])
