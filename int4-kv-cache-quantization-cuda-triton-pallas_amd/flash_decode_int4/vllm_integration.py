@@ -388,12 +388,13 @@ class INT4PagedSequenceCache:
         tokens. Raises before changing the cache when an argument is
         unusable."""
         import torch
-        lens = np.asarray(seq_lens.cpu() if hasattr(seq_lens, "cpu") else seq_lens, np.int64)
-        lens = lens.reshape(-1)
         if torch.cuda.is_current_stream_capturing():
             # The lengths and pages of this call are host data; a replay would
-            # read their transfer buffer again.
+            # read their transfer buffer again. (Before anything else: reading
+            # lengths from the device would end the capture.)
             raise RuntimeError("prefill() cannot be captured into a graph")
+        lens = np.asarray(seq_lens.cpu() if hasattr(seq_lens, "cpu") else seq_lens, np.int64)
+        lens = lens.reshape(-1)
         self._check_prefill(k, v, lens)
         B = k.shape[0]
         self._sync_if_stepped()

@@ -129,18 +129,22 @@ def test_prefill_from_two_streams():
         _check(c, k, k, [n, 600 - n // 2])
 
 
-def test_prefill_is_refused_under_capture():
+@pytest.mark.parametrize("lens_on", ["host", "device"])
+def test_prefill_is_refused_under_capture(lens_on):
+    """The capture around the refused call stays whole, also with lengths on the
+    device (reading those would end it)."""
     import torch
     from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
     c = INT4PagedSequenceCache(8, 2, 64, 2, 64, 16, 64, "float32")
     k = torch.randn(2, 2, 40, 64, device="cuda")
     c.prefill(k, k.clone(), [40, 3])
+    lens = torch.tensor([5, 6], device="cuda") if lens_on == "device" else [5, 6]
     x = torch.zeros(4, device="cuda")
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         x += 1
         with pytest.raises(RuntimeError, match="captured"):
-            c.prefill(k, k, [5, 6])
+            c.prefill(k, k, lens)
     graph.replay()
     torch.cuda.synchronize()
     assert x.tolist() == [1.0] * 4
