@@ -161,7 +161,8 @@ int fdi4_quantize_paged(const float* k, int batch, int max_tokens, int64_t k_bat
 /* Start of sequences 0..batch-1 from dense keys k[b, h, t, :] (float32) and
  * values v[b, h, t, :] (v_in_dtype, converted to the cache's value type as a cast
  * rounds, to nearest even), element strides, channel stride 1, rows starting on
- * 16-byte boundaries, for t < new_lens[b]: the keys as fdi4_quantize_paged writes
+ * 16-byte boundaries, key rows apart (k_row_stride >= head_dim), for
+ * t < new_lens[b]: the keys as fdi4_quantize_paged writes
  * them, the values to their pages, the float32 keys of each sequence's partial
  * last group to k_stage[b, h, 0.., :] (as fdi4_append_paged expects them), new_lens
  * to cache->seq_lens and the used entries of the rows of new_table to

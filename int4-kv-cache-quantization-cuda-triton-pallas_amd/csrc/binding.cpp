@@ -342,7 +342,10 @@ void prefill_paged(torch::Tensor k, torch::Tensor v, torch::Tensor new_lens,
   }
   TORCH_CHECK(cols * k_pages.size(2) >= max_len && cols <= page_table.size(1),
               "new_table must hold the pages of the longest sequence");
-  TORCH_CHECK(k_scale.size(2) * group_rows >= max_len, "k_scale has too few groups");
+  // As the quantizer: the keys as given fit the cache, whatever the lengths.
+  TORCH_CHECK(page_table.size(1) * k_pages.size(2) >= k.size(2),
+              "page_table has too few pages for the key length");
+  TORCH_CHECK(k_scale.size(2) * group_rows >= k.size(2), "k_scale has too few groups");
   CHECK_SAME_DEVICE(k, v);
   CHECK_SAME_DEVICE(k, k_stage);
   CHECK_SAME_DEVICE(k, k_pages);

@@ -516,7 +516,7 @@ int fdi4_prefill_paged(const float* k, int64_t k_batch_stride, int64_t k_head_st
   const int ieb = v_in_dtype == FDI4_V_F32 ? 4 : 2, veb = cache->v_dtype == FDI4_V_F32 ? 4 : 2;
   // 16-byte loads of key and value rows, 16-byte stores of staging rows.
   if (!aligned(k, 16) || k_batch_stride % 4 || k_head_stride % 4 || k_row_stride % 4 ||
-      !aligned(v, 16) || (v_batch_stride * ieb) % 16 || (v_head_stride * ieb) % 16 ||
+      k_row_stride < D || !aligned(v, 16) || (v_batch_stride * ieb) % 16 || (v_head_stride * ieb) % 16 ||
       (v_row_stride * ieb) % 16 || !aligned(k_stage, 16) || st_batch_stride % 4 ||
       st_head_stride % 4 || st_row_stride % 4 || st_row_stride < D)
     return hipErrorInvalidValue;

@@ -187,3 +187,23 @@ def test_failed_prefill_changes_nothing(fails, monkeypatch):
     _check(c, k, v, [150, 33])
     c.prefill(k, v, [100, 140])
     _check(c, k, v, [100, 140])
+
+
+@pytest.mark.parametrize("what", ["tokens", "row_stride"])
+def test_prefill_refuses_what_the_quantizer_refuses(what):
+    """Keys longer than a sequence's pages, whatever the lengths, and key rows
+    that overlap: refused before anything changes."""
+    import torch
+    from flash_decode_int4.vllm_integration import INT4PagedSequenceCache
+    c = INT4PagedSequenceCache(16, 2, 64, 2, 100, 16, 64, "float32")
+    k = torch.randn(2, 2, 40, 64, device="cuda")
+    c.prefill(k, k.clone(), [40, 3])
+    if what == "tokens":
+        bad = torch.randn(2, 2, 200, 64, device="cuda")
+    else:
+        bad = torch.randn(2, 2, 1, 64, device="cuda").expand(2, 2, 40, 64)
+    free = list(c._free)
+    with pytest.raises(RuntimeError):
+        c.prefill(bad, torch.zeros_like(bad), [10, 10])
+    assert c._free == free
+    _check(c, k, k, [40, 3])
