@@ -45,8 +45,9 @@ int chunks_per_seq(const fdi4_paged_cache* c) {
   return c->max_pages * ceil_div(c->page_rows, 16);
 }
 
-int chunks_per_group(const fdi4_paged_cache* c) {
-  return c->pages_per_group * ceil_div(c->page_rows, 16);
+// (64 bits: a group may have any number of pages, more than a sequence has.)
+int64_t chunks_per_group(const fdi4_paged_cache* c) {
+  return (int64_t)c->pages_per_group * ceil_div(c->page_rows, 16);
 }
 
 // Launch-shape overrides set through fdi4_set_tuning (0 = automatic). Atomic
@@ -161,7 +162,7 @@ bool one_wave_per_simd(int d, int v_dtype, int64_t streams) {
 // workgroups of short sequences can be better (B30 Hkv2 Hq8 float32 steps to 6000
 // rows 36.3 -> 37.8).
 int pick_splits(int64_t streams, int waves, int chunks, int d, int v_dtype, bool mfma,
-                bool grouped, bool one_head, int group_chunks) {
+                bool grouped, bool one_head, int64_t group_chunks) {
   const double veb = v_dtype == FDI4_V_F32 ? 4.0 : 2.0;
   const double chunk_bytes = 16.0 * d * (0.5 + veb);
   const double alone = mfma ? (d == 256 ? 1.0 : 0.85) : (d == 256 ? 1.9 : d == 64 ? 0.85 : 1.0);
@@ -197,7 +198,7 @@ int pick_splits(int64_t streams, int waves, int chunks, int d, int v_dtype, bool
 // bits as the append and the decode); with four decode waves its kernel adds
 // four helper waves that re-quantize the open group meanwhile.
 DecodePlan plan_decode(int batch, int hq, int hq_per_kv, int d, int v_dtype, int chunks,
-                       int group_chunks) {
+                       int64_t group_chunks) {
   DecodePlan p;
   p.mfma = use_mfma() ? 1 : 0;
   p.heads_per_wg = p.mfma ? pick_heads_per_wg_mfma(d, hq_per_kv)
@@ -223,7 +224,8 @@ DecodePlan plan_decode(int batch, int hq, int hq_per_kv, int d, int v_dtype, int
     return p;
   }
   p.splits = pick_splits(streams, p.waves, chunks, d, v_dtype, p.mfma != 0,
-                         p.heads_per_wg > 1, hq_per_kv == 1, std::max(1, group_chunks));
+                         p.heads_per_wg > 1, hq_per_kv == 1,
+                         std::max<int64_t>(1, group_chunks));
   return p;
 }
 
@@ -799,7 +801,7 @@ int fdi4_decode_step(const void* query, int query_dtype, int batch, int num_q_he
   // lies in one split): the append fuses into the decode (whose reads of a
   // group's staging rows take 32-bit byte offsets); with several splits the
   // merge follows it.
-  const int group_chunks = chunks_per_group(cache);
+  const int64_t group_chunks = chunks_per_group(cache);
   const bool fused = !a.mfma && a.heads_per_wg == 1 && a.hq_per_kv == 1 &&
                      (a.num_splits == 1 || a.chunks_per_split % group_chunks == 0) &&
                      (int64_t)group_rows * st_row_stride * 4 <= INT32_MAX;

@@ -36,3 +36,17 @@ def test_split_count(head_dim, v_dtype, kv_heads, rep):
                 per_split = -(-chunks // s)
                 assert -(-chunks // per_split) == s
                 assert per_split >= 4
+
+
+@pytest.mark.parametrize("batch,heads,head_dim,rows", [(2, 16, 256, 5000), (5, 16, 256, 2000),
+                                                       (1, 8, 128, 20000)])
+def test_groups_longer_than_any_sequence(batch, heads, head_dim, rows):
+    """One scale group over the whole sequence, however many pages it is said to
+    have (their chunks do not fit 32 bits from 2^27 pages of 256 rows up)."""
+    lib = capi.load()
+    counts = set()
+    for pages in (1 << 20, (1 << 28) + 1, (1 << 31) - 1):
+        cache = capi.PagedCache(max_pages=-(-rows // 256), page_rows=256, num_kv_heads=heads,
+                                head_dim=head_dim, v_dtype=capi.V_F32, pages_per_group=pages)
+        counts.add(lib.fdi4_decode_num_splits(batch, heads, cache))
+    assert len(counts) == 1
