@@ -625,6 +625,12 @@ bool valid_elem_dtype(int dt) {
   return dt == FDI4_K_F32 || dt == FDI4_K_F16 || dt == FDI4_K_BF16;
 }
 
+void set_splits(DecodeArgs* a, int splits, int chunks) {
+  a->num_splits = splits;
+  a->div_splits = fdi4::make_fast_div(splits);
+  a->chunks_per_split = std::max(1, ceil_div(chunks, splits));
+}
+
 int make_decode_args(const void* query, int q_dtype, int batch, int num_q_heads,
                      int64_t q_batch_stride, int64_t q_head_stride,
                      const fdi4_paged_cache* cache, int num_splits, DecodeArgs* a) {
@@ -673,8 +679,8 @@ int make_decode_args(const void* query, int q_dtype, int batch, int num_q_heads,
   a->div_cpp = fdi4::make_fast_div(ceil_div(cache->page_rows, 16));
   a->div_ppg = fdi4::make_fast_div(cache->pages_per_group);
   a->div_hpk = fdi4::make_fast_div(a->hq_per_kv);
-  a->chunks_per_split = std::max(1, ceil_div(chunks, splits));
-  a->num_splits = splits;
+  set_splits(a, splits, chunks);
+  a->turn_splits = a->hq_per_kv == 1 && cache->seq_lens ? 1 : 0;
   a->num_q_heads = num_q_heads;
   a->out = nullptr;
   a->out_dtype = FDI4_K_F32;
@@ -927,10 +933,11 @@ int fdi4_decode_paged_noalloc(const float* query, int batch, int num_q_heads,
   // An automatic count stays within the array (without this, plans of more
   // splits than before would be refused).
   if (num_splits <= 0) {
-    while (a.num_splits > 1 && decode_ws_bytes(batch, num_q_heads, cache->head_dim, a.num_splits) >
-                                   (size_t)FDI4_NOALLOC_SCRATCH_BYTES)
-      --a.num_splits;
-    a.chunks_per_split = std::max(1, ceil_div(chunks_per_seq(cache), a.num_splits));
+    int splits = a.num_splits;
+    while (splits > 1 && decode_ws_bytes(batch, num_q_heads, cache->head_dim, splits) >
+                             (size_t)FDI4_NOALLOC_SCRATCH_BYTES)
+      --splits;
+    set_splits(&a, splits, chunks_per_seq(cache));
   }
   if (!out) return hipErrorInvalidValue;
   const int d = cache->head_dim;

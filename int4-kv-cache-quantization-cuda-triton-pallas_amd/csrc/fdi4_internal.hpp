@@ -127,6 +127,8 @@ struct DecodeArgs {
   int page_rows, pages_per_group, max_pages, hq_per_kv, num_pages;
   FastDiv div_rows, div_cpp, div_ppg, div_hpk;  // by page_rows, 16-row chunks a page,
                                         // pages_per_group, hq_per_kv
+  FastDiv div_splits;                   // by num_splits
+  int turn_splits;                      // 1: splits go round the workgroups (split_of)
   int chunks_per_split, num_splits, num_q_heads;
   int final_out;                        // 1: normalized output; 0: split partials
   int waves;                            // wave64s per workgroup (4 or 8)

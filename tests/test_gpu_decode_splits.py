@@ -56,7 +56,9 @@ CASES = [
     (2, 2, None, 256, [1500, 0], 3, "float16"),       # an empty sequence
     (2, 2, 8, 128, [3000, 1024], 4, None),            # matrix-core grouped kernel
     (1, 2, 16, 64, [2500], 8, "float16"),
-    (2, 2, 4, 256, [1024, 999], 5, None),             # vector grouped kernel (D = 256)
+    (2, 2, 4, 256, [1024, 999], 5, None),             # the same at D = 256
+    (3, 5, None, 64, [2000, 30, 700], 4, None),       # splits in turn over heads, sequences
+    (3, 5, None, 128, [999, 0, 1500], 7, "bfloat16"),
 ]
 
 
