@@ -404,7 +404,9 @@ class INT4PagedSequenceCache:
         need = (lens + self.page_rows - 1) // self.page_rows
         ends = np.cumsum(need).tolist()
         total = ends[-1] if B else 0
-        back = [p for b in range(B) for p in reversed(self._pages[b])]
+        back = []
+        for b in range(B):
+            back.extend(reversed(self._pages[b]))
         own, kept = back[max(0, len(back) - total):], back[:max(0, len(back) - total)]
         cut = len(self._free) - (total - len(own))
         taken = own[::-1] + self._free[cut:][::-1]
