@@ -83,8 +83,6 @@ struct MfmaGeo {
   static constexpr int SZI = D / 2;                // 16-byte items in a scale+zp block
   static constexpr int SZL = (SZI + 63) / 64;      // scale+zp loads per lane
   static constexpr int DIGITS = 6;
-  // Chunks loaded ahead of the one consumed.
-  static constexpr int DEPTH = 1;
   // LDS per wave: the staged scale/zero-point block and the digits of a group
   // while the wave streams, its partial output afterwards.
   static constexpr int kDigBytes = DIGITS * HG * D;
@@ -711,48 +709,43 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
     }
   };
 
-  // One step: (1) rebuild for a new scale group, (2) load the next chunk's scale
-  // block and the chunk DEPTH ahead (past the end one row of the last chunk, so
-  // that every step issues the same loads and the wait counts stay exact),
-  // (3) read the page-table entry of the chunk after that on the scalar unit,
-  // (4) consume chunk c. Called with the DEPTH + 1 buffers in turn, so no
-  // register copy waits on a load.
-  constexpr int DEPTH = G::DEPTH;
+  // One step: (1) rebuild for a new scale group, (2) load the next chunk and its
+  // scale block (past the end one row of the last chunk, so that every step
+  // issues the same loads and the wait counts stay exact), (3) read the
+  // page-table entry of the chunk after that on the scalar unit, (4) consume
+  // chunk c. Called with the two buffers in turn, so no register copy waits on a
+  // load.
   int c = wc0;
   ChunkPos np{};
-  PosMeta mq[DEPTH + 1];      // of chunks c .. c + DEPTH
+  PosMeta cur, next;          // of chunks c and c + 1
   U32x4 sz[G::SZL];
   auto next_meta = [&](int ci) __attribute__((always_inline)) -> PosMeta {
     if (ci < wc1) np = chunk_next(np, cpp, ppg);
     return pos_meta(a, pgm, T, np);
   };
   auto step = [&](Buf& f, Buf& nf) __attribute__((always_inline)) -> bool {
-    if (mq[0].group != cur_group) {
+    if (cur.group != cur_group) {
       rebuild(sz);
-      cur_group = mq[0].group;
+      cur_group = cur.group;
     }
-    load_sz(mq[1], sz);
-    load_chunk(mq[DEPTH], c + DEPTH >= wc1 ? 1 : mq[DEPTH].nval, nf);
-    const PosMeta ahead = next_meta(c + DEPTH + 1);
-    if (mq[0].nval > 0) consume(f, mq[0].nval, false);
-#pragma unroll
-    for (int i = 0; i < DEPTH; ++i) mq[i] = mq[i + 1];
-    mq[DEPTH] = ahead;
+    load_sz(next, sz);
+    load_chunk(next, c + 1 >= wc1 ? 1 : next.nval, nf);
+    const PosMeta ahead = next_meta(c + 2);
+    if (cur.nval > 0) consume(f, cur.nval, false);
+    cur = next;
+    next = ahead;
     c += 1;
     return c >= wc1;
   };
 
   const bool has_work = wc0 < wc1;
-  Buf f[DEPTH + 1];
+  Buf f[2];
   auto first_loads = [&]() __attribute__((always_inline)) {
     np = chunk_pos(a, wc0, cpp);
-    mq[0] = pos_meta(a, pgm, T, np);
-#pragma unroll
-    for (int i = 1; i <= DEPTH; ++i) mq[i] = next_meta(wc0 + i);
-    load_sz(mq[0], sz);
-#pragma unroll
-    for (int i = 0; i < DEPTH; ++i)
-      load_chunk(mq[i], wc0 + i >= wc1 ? 1 : mq[i].nval, f[i]);
+    cur = pos_meta(a, pgm, T, np);
+    next = next_meta(wc0 + 1);
+    load_sz(cur, sz);
+    load_chunk(cur, cur.nval, f[0]);
   };
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -768,14 +761,8 @@ __global__ __launch_bounds__(WAVES * 64) void decode_mfma_kernel(DecodeArgs a) {
   __syncthreads();
   if (has_work) {
     while (true) {
-      if constexpr (DEPTH == 1) {
-        if (step(f[0], f[1])) break;
-        if (step(f[1], f[0])) break;
-      } else {
-        if (step(f[0], f[2])) break;
-        if (step(f[1], f[0])) break;
-        if (step(f[2], f[1])) break;
-      }
+      if (step(f[0], f[1])) break;
+      if (step(f[1], f[0])) break;
     }
   }
 
