@@ -64,6 +64,18 @@ CASES = [
 
 @pytest.mark.parametrize("batch,kv,hq,d,lens,splits,vdt", CASES)
 def test_one_call_equals_two_calls(batch, kv, hq, d, lens, splits, vdt):
+    _one_call_equals_two_calls(batch, kv, hq, d, lens, splits, vdt)
+
+
+@pytest.mark.parametrize("batch,kv,hq,d,lens,splits,vdt", [c for c in CASES if c[2]])
+def test_one_call_equals_two_calls_vector(batch, kv, hq, d, lens, splits, vdt):
+    """The grouped cases on the vector grouped kernel."""
+    from flash_decode_int4 import capi
+    with capi.tuning(decode_vector_only=1):
+        _one_call_equals_two_calls(batch, kv, hq, d, lens, splits, vdt)
+
+
+def _one_call_equals_two_calls(batch, kv, hq, d, lens, splits, vdt):
     import torch
     from flash_decode_int4 import ops
     from flash_decode_int4._lib import load_binding

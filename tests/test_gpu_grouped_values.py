@@ -157,3 +157,19 @@ def test_error_against_float64(D, rep, vdtype):
         a += ((o - e) ** 2).sum().item()
         n += (e ** 2).sum().item()
     assert (a / n) ** 0.5 < 1.5e-7
+
+
+@pytest.mark.parametrize("D,rep,vdtype", [x for x in SHAPES if x[2] != "float32"])
+def test_small_values(D, rep, vdtype):
+    """The matrix cores align a product of a subnormal float16 number as if that
+    were 2^-14, so sums of such values are good to 2^-24 of 2^-14 (a few of these
+    here: the first terms' chunks and the columns); bfloat16 values of any size
+    as any others (units in the last place of float32 sums)."""
+    import torch
+    ops, q, kp, v, s, z, pt, sl = _inputs(D, rep, vdtype, [1000, 77])
+    for scale in (1e-4, 1e-5, 1e-6):
+        x = v * scale if vdtype == "float16" else v * (scale * 1e-30)
+        a = ops.flash_decode_paged(q, kp, x, s, z, pt, sl)
+        b = _exact(q, kp, x, s, z, pt, sl, rep)
+        bound = 4e-7 * b.abs().max().item() + (2.0 ** -36 if vdtype == "float16" else 0.0)
+        assert (a - b).abs().max().item() < bound

@@ -16,10 +16,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,H,rep,D,rows", [(1, 4, 1, 64, 600), (300, 32, 4, 256, 16000),
-                                            (65, 4, 2, 128, 20000)])
+                                            (65, 4, 2, 128, 20000), (33, 8, 4, 256, 16000)])
 def test_automatic_count_fits(B, H, rep, D, rows):
-    """All sequences read the same few pages, so that long tables need little
-    memory; lengths differ."""
+    """Counts that fit (1 and 10 splits), one that is cut to 1 (from 2) and one cut
+    to several (13, 13.6 MB). All sequences read the same few pages, so that long
+    tables need little memory; lengths differ."""
     import torch
     from flash_decode_int4 import capi, ops
     lib = capi.load()
