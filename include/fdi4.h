@@ -84,9 +84,8 @@ typedef struct fdi4_paged_cache {
  * are process-wide and take effect for calls made after fdi4_set_tuning
  * returns; value 0 restores the automatic choice.
  *
- *   FDI4_TUNE_DECODE_VECTOR_ONLY   1: grouped-head decodes at head_dim 64/128
- *                                  run on the vector kernels instead of the
- *                                  int8 matrix-core kernel
+ *   FDI4_TUNE_DECODE_VECTOR_ONLY   1: grouped-head decodes run on the vector
+ *                                  kernels instead of the matrix-core kernel
  *   FDI4_TUNE_DECODE_WAVES         4 or 8 decode wave64s per workgroup (the
  *                                  fused serving step adds 4 re-quantizing
  *                                  waves to 4-wave workgroups, and to 8-wave
@@ -322,7 +321,9 @@ int fdi4_decode_step(const void* query, int query_dtype, int batch, int num_q_he
 
 /* Bytes of the split partials for fdi4_decode_paged_partials: part_acc
  * float [B, Hq, S, D] at offset 0, then part_ml double [B, Hq, S, 2] = (m, l)
- * at offset round_up(B*Hq*S*D*4, 256). */
+ * at offset round_up(B*Hq*S*D*4, 256). acc and l are the sums of
+ * exp(logit - m) * value and of exp(logit - m); m is a shift near the largest
+ * logit, not always that itself, and m = -inf with l = 0 is a split of no rows. */
 size_t fdi4_decode_partials_bytes(int batch, int num_q_heads, int head_dim, int num_splits);
 
 /* The decode kernel alone: writes the per-split partials (the layout of

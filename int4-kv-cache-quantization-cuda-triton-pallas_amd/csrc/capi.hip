@@ -152,15 +152,20 @@ bool one_wave_per_simd(int d, int v_dtype, int64_t streams) {
 //
 // Estimates within 2 % count as equal, and then the count with more workgroups is
 // taken. With one q-head per kv-head a count whose splits hold whole scale groups
-// is preferred by 0.5 us: the serving step appends in the same launch there.
+// is preferred by 0.5 us: the serving step (which takes the decode's count, for
+// the same bits) appends in the same launch there. More is not worth it: the
+// steps that this leaves with a launch of the append are faster than the unsplit
+// ones with the append inside (us a step: B24 H16 T1500 D64 float32 42.8 -> 39.3,
+// T2000 51.4 -> 45.7, B12 H2 D128 T4096 float32 33.6 -> 23.6, B24 H16 D128 T2000
+// float16 63.2 -> 59.7; T1500 50.9 -> 51.2).
 //
 // Measured against the smallest count that gives 2048 waves (us per call): B5 H32
 // T1500 float16 26.3 -> 18.9, B40 H4 T2500 float16 36.9 -> 29.7, B12 H16 D256 T1200
 // float32 54.2 -> 45.3, B3 H32 D256 T2000 float16 38.0 -> 27.9, B40 Hkv4 Hq32 T600
 // float32 24.0 -> 17.0, B6 Hkv8 Hq16 D256 T2500 float16 26.5 -> 19.6. Lengths are
 // not known here: where they are ragged, a count that overfills the CUs with
-// workgroups of short sequences can be better (B30 Hkv2 Hq8 float32 steps to 6000
-// rows 36.3 -> 37.8).
+// workgroups of short sequences can be better (B30 Hkv2 Hq8 D128 float32 steps to
+// 6000 rows 36.7 -> 38.2 us; of equal lengths 54.1 -> 39.3 a decode).
 int pick_splits(int64_t streams, int waves, int chunks, int d, int v_dtype, bool mfma,
                 bool grouped, bool one_head, int64_t group_chunks) {
   const double veb = v_dtype == FDI4_V_F32 ? 4.0 : 2.0;
@@ -169,7 +174,10 @@ int pick_splits(int64_t streams, int waves, int chunks, int d, int v_dtype, bool
   const double rate = (double)streams * chunks * chunk_bytes > 128e6 ? 7.5e6 : 11e6;   // bytes/us
   const bool pairs = waves == 4 && d <= 128 && !(one_head && d == 128 && v_dtype == FDI4_V_F32);
   const int64_t slots = pairs ? 2 * kCUs : kCUs;
-  // At least one chunk a wave in the grouped kernels, four in the per-head one.
+  // At least one chunk a wave in the grouped kernels. Four in the per-head one,
+  // where fewer would be faster for a few short streams (B1 H8 T1024 float16 14.0
+  // us, 9.6 with one chunk a wave): the counts there are ones that callers were
+  // given and rely on (partials of a fixed layout).
   const int per_wave = grouped ? 1 : kMinChunksPerWave;
   const int most = std::max(1, std::min(chunks / (waves * per_wave), kMaxSplits));
   int best = 1;

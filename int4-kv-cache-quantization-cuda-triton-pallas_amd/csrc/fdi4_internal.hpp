@@ -133,7 +133,7 @@ struct DecodeArgs {
   int final_out;                        // 1: normalized output; 0: split partials
   int waves;                            // wave64s per workgroup (4 or 8)
   int heads_per_wg;                     // q-heads per workgroup (1: per-head kernel)
-  int mfma;                             // int8 matrix-core kernel (D = 64 or 128)
+  int mfma;                             // matrix-core kernel (grouped heads)
   void* out;
   int out_dtype;                        // EDtype of out
   int64_t o_b, o_h;
