@@ -176,8 +176,8 @@ int pick_splits(int64_t streams, int waves, int chunks, int d, int v_dtype, bool
   const int64_t slots = pairs ? 2 * kCUs : kCUs;
   // At least one chunk a wave in the grouped kernels. Four in the per-head one,
   // where fewer would be faster for a few short streams (B1 H8 T1024 float16 14.0
-  // us, 9.6 with one chunk a wave): the counts there are ones that callers were
-  // given and rely on (partials of a fixed layout).
+  // us, 9.6 with one chunk a wave): the host contract fixes the counts at such
+  // sizes (tests/test_host_contract.py).
   const int per_wave = grouped ? 1 : kMinChunksPerWave;
   const int most = std::max(1, std::min(chunks / (waves * per_wave), kMaxSplits));
   int best = 1;
